@@ -22,6 +22,13 @@
 // shared groups require E <= 2048.
 // Every load is a global load issued ahead of its use, and the wave sums run on DPP.
 #include "fwht.h"
+#include "shared_rows.h"
+
+#ifndef ROUTER_PIPELINE
+#define ROUTER_PIPELINE moe_router
+#define ROUTER_SHARED_ANY 0  // 1: moe_router_s, the shared expert's rows in any format (moe_router_s.hip)
+#endif
+#define ROUTER_DEFINE(NAME, WG) GD_PIPELINE_NAMED(NAME, WG)  // expands NAME before it is named
 
 #define ROUTER_MAX_TOK 8
 #define ROUTER_MAX_E 4096
@@ -29,11 +36,51 @@
 #define SH_ROWS_PER_GROUP 4
 #define SH_MAX_E 2048  // hidden width covered by the fused shared-expert rows
 
-// Shared expert row 4 sg + w of W_sh (bf16, E columns) on wave w; lane l covers columns
-// 8 l + 512 m (m < E / 512).
 __device__ __forceinline__ float4 rt_f4(gd_u32x4 v) {
     return make_float4(gd_bits_f32(v[0]), gd_bits_f32(v[1]), gd_bits_f32(v[2]), gd_bits_f32(v[3]));
 }
+#if ROUTER_SHARED_ANY
+// Shared row 4 sg + w on wave w: gate row r and up row SF + r, and their SwiGLU.
+template <int KIND>
+__device__ __forceinline__ void router_shared_rows(const GdArgs &a, uint32_t r, uint32_t n_tok, uint32_t E) {
+    const uint32_t lane = threadIdx.x & 63u, SF = a.c[20];
+    const uint8_t *W = gd_buf<const uint8_t>(a, a.c[21]);
+    const uint8_t *const row[2] = {W + (size_t)r * a.c[25], W + (size_t)(SF + r) * a.c[25]};
+    float sum[2][SHR_MAX_TOK];
+    shr_dots<KIND, 2>(row, E, gd_buf<const uint32_t>(a, a.c[0]) + a.c[1], a.c[2], n_tok, sum);
+    float g = 0.f, u = 0.f;
+#pragma unroll
+    for (int t = 0; t < SHR_MAX_TOK; ++t)
+        if ((uint32_t)t < n_tok && lane == (uint32_t)t) {
+            g = sum[0][t];
+            u = sum[1][t];
+        }
+    if (lane < n_tok) gd_buf<float>(a, a.c[22])[a.c[27] + lane * SF + r] = gd_silu_accurate(g) * u;
+}
+// The gate dots g . x[t], one wave per token (w, w + 4): every load of a token in flight together.
+__device__ __forceinline__ void router_shared_gate(const GdArgs &a, uint32_t n_tok, uint32_t E) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t *G = gd_buf<const uint32_t>(a, a.c[23]) + 4u * lane;
+    const uint32_t *X = gd_buf<const uint32_t>(a, a.c[0]) + a.c[1] + 4u * lane;
+    for (uint32_t t = wave; t < n_tok; t += 4u) {
+        float4 gv[ROUTER_MAX_E / 256], xv[ROUTER_MAX_E / 256];
+#pragma unroll
+        for (int m = 0; m < ROUTER_MAX_E / 256; ++m)
+            if (256u * m < E) {
+                gv[m] = rt_f4(*gd_global4(G + 256u * m));
+                xv[m] = rt_f4(*gd_global4(X + t * a.c[2] + 256u * m));
+            }
+        float acc = 0.f;
+#pragma unroll
+        for (int m = 0; m < ROUTER_MAX_E / 256; ++m)
+            if (256u * m < E) acc += (gv[m].x * xv[m].x + gv[m].y * xv[m].y) + (gv[m].z * xv[m].z + gv[m].w * xv[m].w);
+        acc = gd_wave_sum_dpp(acc);
+        if (lane == 0) gd_buf<float>(a, a.c[24])[a.c[28] + t] = acc;
+    }
+}
+#else
+// Shared expert row 4 sg + w of W_sh (bf16, E columns) on wave w; lane l covers columns
+// 8 l + 512 m (m < E / 512).
 __device__ __forceinline__ void router_shared_rows(const GdArgs &a, uint32_t sg, uint32_t n_tok, uint32_t E) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t rows = a.c[20], r = sg * SH_ROWS_PER_GROUP + wave;
@@ -64,8 +111,9 @@ __device__ __forceinline__ void router_shared_rows(const GdArgs &a, uint32_t sg,
         if (lane == 0) H[t * rows + r] = v;
     }
 }
+#endif
 
-GD_PIPELINE_NAMED(moe_router, 256) {
+ROUTER_DEFINE(ROUTER_PIPELINE, 256) {
     __shared__ float red[4][ROUTER_MAX_TOK], reds[4][ROUTER_MAX_TOK];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, row = blockIdx.x;
     const uint32_t x_off = a.c[1], x_stride = a.c[2], E = a.c[7], NE = a.c[6];
@@ -76,6 +124,14 @@ GD_PIPELINE_NAMED(moe_router, 256) {
         // Shared-expert groups follow the router and rotation groups (uniform per group).
         const uint32_t first_sh = NE + E / 128u;
         if (a.c[20] && row >= first_sh) {
+#if ROUTER_SHARED_ANY
+            const uint32_t r = __builtin_amdgcn_readfirstlane((row - first_sh) * SH_ROWS_PER_GROUP + wave);
+            if (row - first_sh >= a.c[20] / SH_ROWS_PER_GROUP) router_shared_gate(a, n_tok, E);
+            else if (a.c[26] == SHR_Q8) router_shared_rows<SHR_Q8>(a, r, n_tok, E);
+            else if (a.c[26] == SHR_F32) router_shared_rows<SHR_F32>(a, r, n_tok, E);
+            else router_shared_rows<SHR_BF16>(a, r, n_tok, E);
+            return;
+#else
             const uint32_t sg = row - first_sh, n_sg = a.c[20] / SH_ROWS_PER_GROUP;
             if (sg < n_sg) {
                 router_shared_rows(a, sg, n_tok, E);
@@ -102,6 +158,7 @@ GD_PIPELINE_NAMED(moe_router, 256) {
                 }
             }
             return;
+#endif
         }
     }
     const float *NW = norm == 2u ? gd_buf<const float>(a, a.c[17]) + a.c[18] : nullptr;

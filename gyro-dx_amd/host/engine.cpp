@@ -835,8 +835,9 @@ class Engine {
     // a multiple of 1024, F 512, top-8; _xg otherwise).
     // Shared expert: a bf16 one of width <= 1024 (a multiple of 256) on E <= 2048 at the _x shapes
     // runs fused into moe_router and moe_decode_down_x; any other (bf16, Q8_0 or fp32, any width
-    // a multiple of 64) runs in the mv kernels first and enters the down kernel as its residual
-    // input, sigmoid(g . x) * W_d (silu(W_g x) * W_u x).
+    // a multiple of 64) runs its gate and up rows in the router's launch (moe_router_s) and its down rows
+    // in moe_decode_shared_down, whose output sigmoid(g . x) * W_d (silu(W_g x) * W_u x) enters the
+    // routed down kernel as its residual input.
     bool decode_supported(const Layer &L, uint32_t n) const {
         if (NE > 256 || n > 8 || E > 4096) return false;
         if (decode_fused_shared(L)) return true;
@@ -888,27 +889,34 @@ class Engine {
                                   "multiple of 128 up to 1024 and top-1..16 (or, for other than uniform TQ2_T "
                                   "experts, E a multiple of 1024 with F 512 and top-8)");
         const bool fused_sh = decode_fused_shared(L);
-        if (L.SF && !fused_sh) {
-            // The shared expert first; its gated output (plus a stack's stream) is the residual
-            // input of the down kernel.
-            const SharedBufs &S = B.shared;
-            shared_expert(L, n, x_uav, x_off, S);
-            dispatch("ew", {S.o, S.o_off, E, S.g, S.g_off, 1, S.s, S.s_off, E, E, n, 4}, (E * n + 255) / 256);
-            if (st.res_uav != kNone)
-                dispatch("ew", {S.s, S.s_off, E, st.res_uav, st.res_off, E, S.s, S.s_off, E, E, n, 2}, (E * n + 255) / 256);
-            st.res_uav = S.s;
-            st.res_off = S.s_off;
-        }
         const uint32_t rsf = fused_sh ? L.SF : 0u;  // shared rows computed inside moe_router
         const uint32_t base_lo = (uint32_t)L.base, base_hi = (uint32_t)(L.base >> 32);
         const bool generic = decode_generic_types(L);
-        dispatch_maybe_timed(bracket == 1, marks, "moe_router",
-                             {x_uav, x_off, E, n, L.router.srv, 0, NE, E, L.has_bias ? L.bias.srv : kNone, 0,
-                              B.logits, B.logits_off, L.has_gate_signs ? L.signs.srv : kNone, 0, B.xh, B.xh_off,
-                              st.on ? (L.has_norm ? 2u : 1u) : 0u, L.has_norm ? L.norm.srv : 0u, 0,
-                              bits(L.norm_eps), 2 * rsf, rsf ? L.sh_gu.srv : 0u, rsf ? B.sh_h : 0u,
-                              rsf ? L.sh_gate.srv : 0u, rsf ? B.sh_g : 0u},
-                             NE + E / 128 + (rsf ? 2 * rsf / 4 + 1 : 0));
+        if (L.SF && !fused_sh) {
+            // The shared expert's SwiGLU rows and gate dots in the router's launch, its gated output (plus
+            // a stack's stream) in a launch of its own: the residual input of the down kernel.
+            const SharedBufs &S = B.shared;
+            dispatch_maybe_timed(bracket == 1, marks, "moe_router_s",
+                                 {x_uav, x_off, E, n, L.router.srv, 0, NE, E, L.has_bias ? L.bias.srv : kNone, 0,
+                                  B.logits, B.logits_off, L.has_gate_signs ? L.signs.srv : kNone, 0, B.xh, B.xh_off,
+                                  0, 0, 0, 0, L.SF, L.sh_gu.srv, S.a, L.sh_gate.srv, S.g, L.sh_row_e, L.sh_kind, S.a_off,
+                                  S.g_off},
+                                 NE + E / 128 + L.SF / 4 + 1);
+            dispatch("moe_decode_shared_down",
+                     {S.a, S.a_off, S.g, S.g_off, L.sh_down.srv, L.sh_row_f, L.sh_kind, L.SF, E, n, S.s, S.s_off,
+                      st.res_uav != kNone ? 1u : 0u, st.res_uav != kNone ? st.res_uav : 0u, st.res_off},
+                     (E + 7) / 8);
+            st.res_uav = S.s;
+            st.res_off = S.s_off;
+        } else {
+            dispatch_maybe_timed(bracket == 1, marks, "moe_router",
+                                 {x_uav, x_off, E, n, L.router.srv, 0, NE, E, L.has_bias ? L.bias.srv : kNone, 0,
+                                  B.logits, B.logits_off, L.has_gate_signs ? L.signs.srv : kNone, 0, B.xh, B.xh_off,
+                                  st.on ? (L.has_norm ? 2u : 1u) : 0u, L.has_norm ? L.norm.srv : 0u, 0,
+                                  bits(L.norm_eps), 2 * rsf, rsf ? L.sh_gu.srv : 0u, rsf ? B.sh_h : 0u,
+                                  rsf ? L.sh_gate.srv : 0u, rsf ? B.sh_g : 0u},
+                                 NE + E / 128 + (rsf ? 2 * rsf / 4 + 1 : 0));
+        }
         if (!generic || !decode_generic_tuned()) {
             if (!generic && decode_tuned_tq2()) {
                 // One token: the build that holds a block's activations in registers at once;
@@ -1239,10 +1247,8 @@ class Engine {
         B.shared = {};
         if (L.SF && !decode_fused_shared(L)) {
             SharedBufs &S = B.shared;
-            S.h = S.a = S.o = S.g = S.s = na_base.uav;
-            S.h_off = take((uint64_t)n * 2 * L.SF * 4);
+            S.a = S.g = S.s = na_base.uav;
             S.a_off = take((uint64_t)n * L.SF * 4);
-            S.o_off = take((uint64_t)n * E * 4);
             S.g_off = take((uint64_t)n * 4);
             S.s_off = take((uint64_t)n * E * 4);
         }
