@@ -1,7 +1,8 @@
 // Points entries of the context's table of base pointers at addresses carried in the dispatch's
-// constants, so that work queued on a stream can name memory known only when it is queued (the
-// caller's input and output of the MoE engine's no-allocation entry point) without a host copy
-// into the table. Vector stores only; the next dispatch sees the entries.
+// constants, so that a caller of gd_dispatch_on whose kernels take table indices can name memory known
+// only when the work is queued without a host copy into the table (the MoE engine's own decode kernels
+// carry such addresses in their constants instead: gd_buf_at). Vector stores only; the next dispatch
+// sees the entries.
 // Constants: 0 count (at most 19), then for entry i: 1 + 3 i table index, 2 + 3 i address bits
 // 0..31, 3 + 3 i address bits 32..63. Indices at or past the table's 65,536 entries are skipped.
 #include "gd_kernel.h"

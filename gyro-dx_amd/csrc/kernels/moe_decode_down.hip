@@ -15,7 +15,7 @@
 // Grid: x = E / 8, y = n_tok; 512 threads.
 // Constants: 0 gu_uav 1 gu_off 2 ids_uav 3 ids_off 4 weights_uav 5 weights_off 6 base_lo
 // 7 base_hi 8 slot_stride 9 down_off (bytes from an expert's bundle start) 10 codebook_srv
-// 11 signs_srv (0xffffffff: none) 12 signs_off 13 out_uav 14 out_off 15 E 16 F 17 n_used
+// 11 signs_srv (0xffffffff: none) 12 signs_off 13 out_uav (or its address in 58, 59) 14 out_off 15 E 16 F 17 n_used
 // 18 n_tok 19 parts 20 n_expert 21 residual (0: none, 1: add) 22 res_uav 23 res_off: with the
 // residual each output adds res[t][row] after the combine (the residual step of a stack; res
 // may alias out). Constants past the caller's count read zero, so a 21-constant dispatch has
@@ -176,6 +176,6 @@ GD_PIPELINE_NAMED(moe_decode_down, 512) {
     if (lane == 0u) {
         const uint32_t orow = row0 + wave;
         if (a.c[21]) acc = gd_buf<const float>(a, a.c[22])[a.c[23] + t * E + orow] + acc;
-        gd_buf<float>(a, a.c[13])[a.c[14] + t * E + orow] = acc;
+        gd_buf_at<float, GD_OUT_ADDR>(a, a.c[13])[a.c[14] + t * E + orow] = acc;
     }
 }

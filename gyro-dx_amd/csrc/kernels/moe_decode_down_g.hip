@@ -20,7 +20,7 @@
 // Grid: x = E / R, y = n_tok; 512 threads.
 // Constants: 0 act_uav 1 act_off (act[(t U + k) F + f], from moe_decode_gu_g) 2 ids_uav 3 ids_off
 // 4 weights_uav 5 weights_off 6 base_lo 7 base_hi 8 slot_stride 9 down_off 10 codebook_srv
-// 11 signs_srv (0xffffffff: none) 12 signs_off 13 out_uav 14 out_off 15 E 16 F 17 n_used
+// 11 signs_srv (0xffffffff: none) 12 signs_off 13 out_uav (or its address in 58, 59) 14 out_off 15 E 16 F 17 n_used
 // 18 n_tok 19 R 20 n_expert 21 residual 22 res_uav 23 res_off (24 xtab_srv: the generic form).
 // Requires TQ2_T experts (any types in the generic form), F a multiple of 128 up to 1024,
 // 1 <= n_used <= 16, n_used F / 128 <= DG_MAX_ABLK, n_used F / 64 ceil(R / 2) <= 512 DG_ITEMS
@@ -80,7 +80,7 @@ DG_DEFINE(DG_PIPELINE, 512) {
     // The output row's address and its residual now, not after the sums: there they would add
     // two table reads and a load to the end of the group. Without a residual the output row is
     // read instead, and not used.
-    float *OUT = gd_buf<float>(a, a.c[13]) + a.c[14];
+    float *OUT = gd_buf_at<float, GD_OUT_ADDR>(a, a.c[13]) + a.c[14];
     const bool residual = a.c[21] != 0u;
     const float *RES = residual ? gd_buf<const float>(a, a.c[22]) + a.c[23] : OUT;
     // Lane k of 16-lane row q stores output row q (see the row sums below).

@@ -20,7 +20,7 @@
 // Grid: x = E / R, y = n_tok; 512 threads.
 // Constants: 0 gu_uav 1 gu_off 2 ids_uav 3 ids_off 4 weights_uav 5 weights_off 6 xtab_srv
 // 7 (unused) 8 (unused) 9 (unused) 10 codebook_srv 11 signs_srv (0xffffffff: none) 12 signs_off
-// 13 out_uav 14 out_off 15 E 16 F 17 n_used 18 n_tok 19 parts 20 n_expert 21 residual (0: none,
+// 13 out_uav (or its address in 58, 59) 14 out_off 15 E 16 F 17 n_used 18 n_tok 19 parts 20 n_expert 21 residual (0: none,
 // 1: add) 22 res_uav 23 res_off 24 shared (0: none, 1: the layer's shared expert) 25 sh_h_uav
 // (fp32 [n][2 SF]: W_sg x then W_su x, from moe_router) 26 (unused) 27 shg_uav (g . x [n])
 // 28 shg_off 29 sh_down_srv (bf16 [E][SF]) 30 SF (<= 1024, a multiple of 256). The shared
@@ -305,6 +305,6 @@ DX_DEFINE(DX_PIPELINE, 512) {
             acc += g * shs[tid];
         }
         if (a.c[21]) acc = res_v + acc;
-        gd_buf<float>(a, a.c[13])[a.c[14] + t * E + row0 + tid] = acc;
+        gd_buf_at<float, GD_OUT_ADDR>(a, a.c[13])[a.c[14] + t * E + row0 + tid] = acc;
     }
 }

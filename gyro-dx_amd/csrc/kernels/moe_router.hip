@@ -16,7 +16,7 @@
 // without weight, 2: with weight; zero when the caller passes 16 constants) 17 norm_w_srv
 // 18 norm_w_off 19 eps (fp32 bits) 20 shared rows (2 SF; 0: no shared expert) 21 sh_w_srv (bf16
 // [2 SF][E]: gate rows then up rows) 22 sh_h_uav (fp32 [n][2 SF]) 23 sh_gate_srv (fp32 [E])
-// 24 sh_g_uav (fp32 [n]). With a shared expert (src/engine.zig:644-653) the grid has 2 SF / 4 + 1
+// 24 sh_g_uav (fp32 [n]) 56, 57 address of x (0: entry 0's). With a shared expert (src/engine.zig:644-653) the grid has 2 SF / 4 + 1
 // further groups after the n_expert + E / 128 above: each of the first computes 4 bf16 rows
 // (one per wave) of W_sg x and W_su x on the unrotated input, the last the gate dot g . x. The
 // shared groups require E <= 2048.
@@ -47,7 +47,7 @@ __device__ __forceinline__ void router_shared_rows(const GdArgs &a, uint32_t r, 
     const uint8_t *W = gd_buf<const uint8_t>(a, a.c[21]);
     const uint8_t *const row[2] = {W + (size_t)r * a.c[25], W + (size_t)(SF + r) * a.c[25]};
     float sum[2][SHR_MAX_TOK];
-    shr_dots<KIND, 2>(row, E, gd_buf<const uint32_t>(a, a.c[0]) + a.c[1], a.c[2], n_tok, sum);
+    shr_dots<KIND, 2>(row, E, gd_buf_at<const uint32_t, GD_IN_ADDR>(a, a.c[0]) + a.c[1], a.c[2], n_tok, sum);
     float g = 0.f, u = 0.f;
 #pragma unroll
     for (int t = 0; t < SHR_MAX_TOK; ++t)
@@ -61,7 +61,7 @@ __device__ __forceinline__ void router_shared_rows(const GdArgs &a, uint32_t r, 
 __device__ __forceinline__ void router_shared_gate(const GdArgs &a, uint32_t n_tok, uint32_t E) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t *G = gd_buf<const uint32_t>(a, a.c[23]) + 4u * lane;
-    const uint32_t *X = gd_buf<const uint32_t>(a, a.c[0]) + a.c[1] + 4u * lane;
+    const uint32_t *X = gd_buf_at<const uint32_t, GD_IN_ADDR>(a, a.c[0]) + a.c[1] + 4u * lane;
     for (uint32_t t = wave; t < n_tok; t += 4u) {
         float4 gv[ROUTER_MAX_E / 256], xv[ROUTER_MAX_E / 256];
 #pragma unroll
@@ -86,7 +86,7 @@ __device__ __forceinline__ void router_shared_rows(const GdArgs &a, uint32_t sg,
     const uint32_t rows = a.c[20], r = sg * SH_ROWS_PER_GROUP + wave;
     if (r >= rows) return;  // uniform per wave; no barrier follows
     const uint32_t *Wsh = gd_buf<const uint32_t>(a, a.c[21]) + ((size_t)r * E + 8u * lane) / 2u;
-    const uint32_t *X = gd_buf<const uint32_t>(a, a.c[0]) + a.c[1] + 8u * lane;
+    const uint32_t *X = gd_buf_at<const uint32_t, GD_IN_ADDR>(a, a.c[0]) + a.c[1] + 8u * lane;
     float *H = gd_buf<float>(a, a.c[22]);
     constexpr int MM = SH_MAX_E / 512;  // column chunks
     gd_u32x4 w[MM];
@@ -119,7 +119,7 @@ ROUTER_DEFINE(ROUTER_PIPELINE, 256) {
     const uint32_t x_off = a.c[1], x_stride = a.c[2], E = a.c[7], NE = a.c[6];
     const uint32_t n_tok = a.c[3] < ROUTER_MAX_TOK ? a.c[3] : ROUTER_MAX_TOK;
     const uint32_t norm = a.c[16];
-    const float *X = gd_buf<const float>(a, a.c[0]);
+    const float *X = gd_buf_at<const float, GD_IN_ADDR>(a, a.c[0]);
     {
         // Shared-expert groups follow the router and rotation groups (uniform per group).
         const uint32_t first_sh = NE + E / 128u;

@@ -21,7 +21,7 @@ SYMBOLS = [
     "gd_barrier", "gd_timestamp", "gd_submit", "gd_wait_compute", "gd_read_timestamps",
     "gd_queue_wait_storage", "gd_read_ranges_after", "gd_release_buffer", "gd_release_file", "gd_destroy",
     # Extensions without a counterpart in the reference ABI: timed dispatch for profiling, and the
-    # stream launch and caller-memory table entries of the MoE engine's no-allocation entry point.
+    # stream launch and scratch-array table entries of the MoE engine's no-allocation entry point.
     "gd_dispatch_timed", "gd_dispatch_on", "gd_wrap_memory",
 ]
 

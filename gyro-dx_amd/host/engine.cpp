@@ -301,7 +301,8 @@ class Engine {
     // Direct launches (no recording) on a caller's stream, for gm_forward_decode_noalloc.
     bool direct = false;
     void *direct_stream = nullptr;
-    Buffer na_base, na_shh, na_shg, na_x, na_out;  // table entries into `scratch` and for the caller's x, out
+    uint64_t direct_x = 0, direct_out = 0;  // the caller's x and out, carried in the constants
+    Buffer na_base, na_shh, na_shg;         // table entries into `scratch`
     // Compute units of the device (the persistent GEMM's two groups per unit, the decode
     // kernels' target group count).
     uint32_t cus = 0;
@@ -380,9 +381,15 @@ class Engine {
     }
 
     void dispatch_words(const char *name, const uint32_t *c, uint32_t count, uint32_t x, uint32_t y, uint32_t z) {
-        if (direct)
-            check(gd_dispatch_on(dev.ctx, pipe(name), c, count, x, y, z, direct_stream), "gd_dispatch_on");
-        else
+        if (direct) {
+            // Constants 56 to 59: the addresses of the caller's input and output (gd_buf_at), read by
+            // the router and down kernels in the place of a table entry.
+            uint32_t words[60] = {};
+            std::memcpy(words, c, count * sizeof(uint32_t));
+            std::memcpy(words + 56, &direct_x, 8);
+            std::memcpy(words + 58, &direct_out, 8);
+            check(gd_dispatch_on(dev.ctx, pipe(name), words, 60, x, y, z, direct_stream), "gd_dispatch_on");
+        } else
             dev.dispatch(pipe(name), c, count, x, y, z);
     }
     void dispatch(const char *name, const std::vector<uint32_t> &c, uint32_t x, uint32_t y = 1, uint32_t z = 1) {
@@ -468,14 +475,11 @@ class Engine {
         }
         range_flag = dev.buffer(256, Kind::device);
         fill_zero(range_flag);
-        // Table entries of the no-allocation entry point: into this GPU's scratch array, and two
-        // whose addresses each call sets (the caller's input and output).
+        // Table entries of the no-allocation entry point, into this GPU's scratch array.
         uint8_t *sp = static_cast<uint8_t *>(scratch_address(adapter));
         na_base = dev.wrap(sp, GM_NOALLOC_SCRATCH_BYTES);
         na_shh = dev.wrap(sp + kNoallocShH, kNoallocShHBytes);
         na_shg = dev.wrap(sp + kNoallocShG, kNoallocShGBytes);
-        na_x = dev.wrap(nullptr, 0);
-        na_out = dev.wrap(nullptr, 0);
         int cu = 0;
         if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, (int)adapter) != hipSuccess) cu = 0;
         cus = (uint32_t)std::max(cu, 0);
@@ -1262,12 +1266,12 @@ class Engine {
             ~Restore() {
                 e->direct = false;
                 e->direct_stream = nullptr;
+                e->direct_x = e->direct_out = 0;
             }
         } restore{this};
-        const uint64_t xa = (uint64_t)(uintptr_t)x, ya = (uint64_t)(uintptr_t)y;
-        dispatch("gd_table_set",
-                 {2u, na_x.uav, (uint32_t)xa, (uint32_t)(xa >> 32), na_out.uav, (uint32_t)ya, (uint32_t)(ya >> 32)}, 1);
-        ffn_decode(il, n, na_x.uav, 0, na_out.uav, 0, 0, nullptr, StackStep{}, &B);
+        direct_x = (uint64_t)(uintptr_t)x;
+        direct_out = (uint64_t)(uintptr_t)y;
+        ffn_decode(il, n, 0, 0, 0, 0, 0, nullptr, StackStep{}, &B);
     }
 
     void forward(uint32_t il, uint32_t path, const float *x, uint32_t n, float *y) {

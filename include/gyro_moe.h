@@ -137,9 +137,9 @@ GM_API int gm_read_outputs(gm_engine *e, float *out, uint32_t n_total);
  * `stream` (a hipStream_t of the engine's device; NULL: the engine's compute stream) without
  * waiting for it. It calls no hipMalloc / hipFree and no memset or copy: router logits, routes,
  * the rotated input, the gate/up partials and the shared expert's rows live in a fixed device
- * array of GM_NOALLOC_SCRATCH_BYTES per GPU, and a small kernel points two table entries at x and
- * out. A layer shape whose buffers exceed that array is refused with an error. Every call on one
- * GPU shares the array and those two entries: calls that overlap on one GPU race, so a caller
+ * array of GM_NOALLOC_SCRATCH_BYTES per GPU, and the launches carry the addresses of x and out in
+ * their constants. A layer shape whose buffers exceed that array is refused with an error. Every call on one
+ * GPU shares the array: calls that overlap on one GPU race, so a caller
  * serialises them (one stream, or its own ordering). Results equal gm_forward's bit for bit: the
  * decode path keeps its activations in fp32, so no call of it is ever recomputed on another path
  * (the binary16 range recompute of gm_forward concerns GM_PATH_PREFILL only). */
