@@ -22,6 +22,7 @@
 #include <string>
 #include <vector>
 
+#include "copy_pool.h"
 #include "device.h"
 #include "gyro_moe.h"
 
@@ -350,7 +351,7 @@ class Engine {
     uint32_t slot_stride = 0, per_arena = 0, used_slots = 0;
     Buffer lookup;
     // Shared buffers.
-    Buffer staging, codebook, zeros;
+    Buffer staging, status, codebook, zeros;
     Buffer x_in, router_out, ids, weights, table, xh, gu, gu_part, act, down, out;
     Buffer order, meta;  // prefill: sorted slots; segment starts, tile count and tile list
     // Prefill: per chunk of 256 slots, the slots that chose each expert ([chunk][n_expert]; the
@@ -425,24 +426,138 @@ class Engine {
         closedir(d);
     }
 
-    // Copies host bytes into a device buffer through the mapped staging buffer and the
-    // bit-exact copy of the elementwise pipeline (as src/gpu_engine.zig:447-461 uploads the
-    // codebook).
-    void upload(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes) {
+    // Host transfers go through the mapped staging buffer in slots of kSlotBytes, copied to and from
+    // device memory by the transfer kernel on the compute stream. A slot is reused once the submission
+    // that last touched it (slot_ticket) has finished; slots of the open recording are in `open_slots`
+    // until its submission names their ticket.
+    static constexpr uint64_t kSlotBytes = 2u << 20;
+    static constexpr uint32_t kSlots = kStagingBytes / (2u << 20);
+    uint64_t slot_ticket[kSlots] = {};
+    uint32_t next_slot = 0;
+    std::vector<uint32_t> open_slots;
+    CopyPool copies;
+
+    uint32_t take_slot() {
+        const uint32_t s = next_slot;
+        next_slot = (next_slot + 1) % kSlots;
+        if (slot_ticket[s]) dev.wait(slot_ticket[s]);
+        slot_ticket[s] = 0;
+        open_slots.push_back(s);
+        return s;
+    }
+    uint64_t submit() {
+        const uint64_t ticket = dev.submit();
+        for (uint32_t s : open_slots) slot_ticket[s] = ticket;
+        open_slots.clear();
+        return ticket;
+    }
+    static uint32_t transfer_groups(uint32_t words) { return std::max(1u, (words + 4095) / 4096); }
+
+    // Records the copy of at most kSlotBytes host bytes into a device buffer (a recording is open).
+    void record_upload(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes) {
+        const uint32_t s = take_slot(), words = (uint32_t)(bytes / 4), at = (uint32_t)(s * (kSlotBytes / 4));
+        copies.copy(staging.mapped + s * kSlotBytes, src, bytes);
+        dispatch("transfer", {staging.uav, at, dst.uav, (uint32_t)(dst_off / 4), words}, transfer_groups(words));
+    }
+    // Size of the parts a transfer of `bytes` goes in: the host's copies and the link's overlap from part
+    // to part, but a part's submission costs the host about 8 us.
+    static uint64_t part_bytes(uint64_t bytes) {
+        const uint64_t p = (bytes / 6 + 4095) & ~uint64_t(4095);
+        return std::min(kSlotBytes, std::max<uint64_t>(p, 512u << 10));
+    }
+    // Copies host bytes into a device buffer. All but the last part go out in submissions of their own, so
+    // that the host fills the next slot while the link moves this one; the last is left in an open
+    // recording (begin_upload), submitted (upload_later: for data that only this stream reads before
+    // the next wait) or submitted and waited for (upload). The source is read before any returns.
+    void begin_upload(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes) {
         if (bytes % 4 || dst_off % 4) throw NativeError(-1, "upload must be word aligned");
         const uint8_t *s = static_cast<const uint8_t *>(src);
-        while (bytes) {
-            const uint64_t chunk = std::min<uint64_t>(bytes, kStagingBytes);
-            std::memcpy(staging.mapped, s, chunk);
-            const uint32_t words = (uint32_t)(chunk / 4);
+        const uint64_t part = part_bytes(bytes);
+        for (; bytes > part; bytes -= part, s += part, dst_off += part) {
             dev.begin();
-            dispatch("ew", {staging.uav, 0, 0, staging.uav, 0, 0, dst.uav, (uint32_t)(dst_off / 4), 0, words, 1, 5},
-                     (words + 255) / 256);
-            dev.wait(dev.submit());
-            s += chunk;
-            dst_off += chunk;
-            bytes -= chunk;
+            record_upload(dst, dst_off, s, part);
+            submit();
         }
+        dev.begin();
+        if (bytes) record_upload(dst, dst_off, s, bytes);
+    }
+    uint64_t upload_later(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes) {
+        begin_upload(dst, dst_off, src, bytes);
+        return submit();
+    }
+    void upload(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes) {
+        dev.wait(upload_later(dst, dst_off, src, bytes));
+    }
+
+    // The flag words a prefill submission leaves, as the transfer kernel gathered them.
+    struct Flags {
+        uint32_t gemm_error = 0, range = 0;
+    };
+    void record_flags() {
+        dispatch("transfer", {0, 0, 0, 0, 0, 3, status.uav, 0, gemm_sched.uav, 1, range_flag.uav, 0, meta.uav, kMetaRangeFlag}, 1);
+    }
+    Flags flags() const { return {status.words()[0], status.words()[1] | status.words()[2]}; }  // after the wait
+
+    // Ends the open recording with the copy of `bytes` of a device buffer to host memory (and, with
+    // want_flags, of the flag words): the first part in this submission, later ones in their own,
+    // kAhead ahead of the part whose copy out of its staging slot is handed on next. Returns the flags;
+    // with any set, the host memory is not written.
+    Flags finish_download(const Buffer &src, void *dst, uint64_t bytes, bool want_flags) {
+        struct Part {
+            uint64_t ticket;
+            uint32_t slot, bytes;
+        };
+        // At most kBatch slots wait for their copies and kAhead are being filled, so no slot comes round
+        // to a new part before its copy is made.
+        constexpr uint32_t kAhead = 4, kBatch = 8;
+        static_assert(kAhead + kBatch <= kSlots, "slots of a download");
+        const uint64_t step = part_bytes(bytes);
+        const uint32_t parts = (uint32_t)((bytes + step - 1) / step);
+        // All threads on one part until it is out; from a dozen parts on one thread on each, which a fresh
+        // output in 2 MB pages needs: a page is cleared by the first thread that touches it while
+        // the others wait (32 MB: 2.3 ms in small pieces, 0.75 ms in whole parts).
+        const uint64_t piece = parts >= 12 ? step : CopyPool::kPiece;
+        std::vector<Part> part(parts);
+        auto issue = [&](uint32_t i) {
+            if (i) dev.begin();
+            part[i].bytes = (uint32_t)std::min<uint64_t>(step, bytes - i * step);
+            part[i].slot = take_slot();
+            const uint32_t words = part[i].bytes / 4, at = (uint32_t)(part[i].slot * (kSlotBytes / 4));
+            if (i == 0 && want_flags)
+                dispatch("transfer", {src.uav, 0, staging.uav, at, words, 3, status.uav, 0, gemm_sched.uav, 1,
+                                      range_flag.uav, 0, meta.uav, kMetaRangeFlag},
+                         transfer_groups(words));
+            else
+                dispatch("transfer", {src.uav, (uint32_t)(i * (step / 4)), staging.uav, at, words}, transfer_groups(words));
+            part[i].ticket = submit();
+        };
+        Flags f;
+        issue(0);
+        for (uint32_t i = 0, issued = 1; i < parts; ++i) {
+            for (; issued < parts && issued < i + kAhead; ++issued) issue(issued);
+            dev.wait(part[i].ticket);
+            if (i == 0 && want_flags) {
+                f = flags();
+                if (f.gemm_error || f.range) {
+                    dev.wait(part[issued - 1].ticket);
+                    return f;
+                }
+            }
+            uint8_t *to = static_cast<uint8_t *>(dst) + i * step;
+            const uint8_t *from = staging.mapped + part[i].slot * kSlotBytes;
+            if (parts == 1) {
+                copies.copy(to, from, part[i].bytes);
+            } else {
+                copies.post(to, from, part[i].bytes, piece);
+                if ((i + 1) % kBatch == 0 || i + 1 == parts) copies.finish();
+            }
+        }
+        return f;
+    }
+    void download(const Buffer &src, void *dst, uint64_t bytes) {
+        if (!bytes) throw NativeError((gd_result)0x80070057u, "an empty read");  // E_INVALIDARG, as gd_readback
+        dev.begin();
+        finish_download(src, dst, bytes, false);
     }
 
     void fill_zero(const Buffer &dst) {
@@ -463,6 +578,7 @@ class Engine {
         dev.init(adapter);
         load_kernels(kernel_dir);
         staging = dev.buffer(kStagingBytes, Kind::host);
+        status = dev.buffer(256, Kind::host);
         zeros = dev.buffer(1u << 18, Kind::host);  // stays zero: the source of fills
         codebook = dev.buffer(8192, Kind::device);
         std::vector<uint8_t> book = read_file(kernel_dir + "/../../data/gyro_codebook.f16");
@@ -605,9 +721,9 @@ class Engine {
                 arenas.push_back(dev.buffer((uint64_t)per_arena * slot_stride + 256, Kind::device));
             const uint64_t off = (uint64_t)(slot % per_arena) * slot_stride;
             const Buffer &arena = arenas[ai];
-            upload(arena, off, d.gate[e], gb[e]);
-            upload(arena, off + gb[e], d.up[e], ub[e]);
-            upload(arena, off + gb[e] + ub[e], d.down[e], db[e]);
+            upload_later(arena, off, d.gate[e], gb[e]);
+            upload_later(arena, off + gb[e], d.up[e], ub[e]);
+            upload_later(arena, off + gb[e] + ub[e], d.down[e], db[e]);
             L.max_scale = std::max({L.max_scale, max_block_scale(d.gate[e], gb[e], block_bytes_of(d.types[e * 3])),
                                     max_block_scale(d.up[e], ub[e], block_bytes_of(d.types[e * 3 + 1])),
                                     max_block_scale(d.down[e], db[e], block_bytes_of(d.types[e * 3 + 2]))});
@@ -620,18 +736,18 @@ class Engine {
             if (e == 0) L.base = desc[0].gate;
         }
         L.xtab = dev.buffer(NE * sizeof(ExpertDesc), Kind::device);
-        upload(L.xtab, 0, desc.data(), NE * sizeof(ExpertDesc));
+        upload_later(L.xtab, 0, desc.data(), NE * sizeof(ExpertDesc));
         L.router = dev.buffer((uint64_t)NE * E * 4, Kind::device);
-        upload(L.router, 0, d.router, (uint64_t)NE * E * 4);
+        upload_later(L.router, 0, d.router, (uint64_t)NE * E * 4);
         if (NE <= 256 && E % 256 == 0) {  // the prefill path's router shapes
             const std::vector<uint32_t> sp = split_router_rows(d.router, NE, E);
             L.router16 = dev.buffer(sp.size() * 4, Kind::device);
-            upload(L.router16, 0, sp.data(), sp.size() * 4);
+            upload_later(L.router16, 0, sp.data(), sp.size() * 4);
         }
         if (d.router_bias) {
             L.has_bias = true;
             L.bias = dev.buffer(NE * 4, Kind::device);
-            upload(L.bias, 0, d.router_bias, NE * 4);
+            upload_later(L.bias, 0, d.router_bias, NE * 4);
         }
         std::vector<float> signs(E + F, 1.0f);
         if (d.gate_signs) {
@@ -643,11 +759,11 @@ class Engine {
             std::memcpy(signs.data() + E, d.down_signs, F * 4);
         }
         L.signs = dev.buffer((E + F) * 4, Kind::device);
-        upload(L.signs, 0, signs.data(), (E + F) * 4);
+        upload_later(L.signs, 0, signs.data(), (E + F) * 4);
         if (d.norm_weight) {
             L.has_norm = true;
             L.norm = dev.buffer((uint64_t)E * 4, Kind::device);
-            upload(L.norm, 0, d.norm_weight, (uint64_t)E * 4);
+            upload_later(L.norm, 0, d.norm_weight, (uint64_t)E * 4);
         }
         if (!(d.norm_eps >= 0.0f)) throw NativeError(-1, "norm_eps must be a non-negative number");
         L.norm_eps = d.norm_eps;
@@ -667,19 +783,19 @@ class Engine {
                 // Raw GGUF blocks into a temporary buffer, then q8_repack into the mv_q8 layout
                 // (src/gpu_engine.zig:289-306).
                 Buffer raw = dev.buffer(std::max(2 * SF * src_e, (uint64_t)E * src_f), Kind::device);
-                upload(raw, 0, d.sh_gate, SF * src_e);
-                upload(raw, SF * src_e, d.sh_up, SF * src_e);
+                upload_later(raw, 0, d.sh_gate, SF * src_e);
+                upload_later(raw, SF * src_e, d.sh_up, SF * src_e);
                 repack_q8(raw, 2 * SF, E, L.sh_gu, L.sh_row_e);
-                upload(raw, 0, d.sh_down, (uint64_t)E * src_f);
+                upload_later(raw, 0, d.sh_down, (uint64_t)E * src_f);
                 repack_q8(raw, E, SF, L.sh_down, L.sh_row_f);
                 dev.release(raw);
             } else {
-                upload(L.sh_gu, 0, d.sh_gate, SF * src_e);
-                upload(L.sh_gu, SF * src_e, d.sh_up, SF * src_e);
-                upload(L.sh_down, 0, d.sh_down, (uint64_t)E * src_f);
+                upload_later(L.sh_gu, 0, d.sh_gate, SF * src_e);
+                upload_later(L.sh_gu, SF * src_e, d.sh_up, SF * src_e);
+                upload_later(L.sh_down, 0, d.sh_down, (uint64_t)E * src_f);
             }
             L.sh_gate = dev.buffer((uint64_t)E * 4, Kind::device);
-            upload(L.sh_gate, 0, d.sh_gate_inp, (uint64_t)E * 4);
+            upload_later(L.sh_gate, 0, d.sh_gate_inp, (uint64_t)E * 4);
             // Binary16 copies for the prefill GEMMs, each matrix scaled by its own power of two.
             const uint64_t half = SF * E * 2;
             std::vector<float> fl;
@@ -687,14 +803,14 @@ class Engine {
             L.sh_gu16 = dev.buffer(2 * half, Kind::device);
             shared_to_floats(kind, d.sh_gate, SF, E, fl);
             L.sh_unscale[0] = floats_to_scaled_half(fl.data(), fl.size(), h16);
-            upload(L.sh_gu16, 0, h16.data(), half);
+            upload_later(L.sh_gu16, 0, h16.data(), half);
             shared_to_floats(kind, d.sh_up, SF, E, fl);
             L.sh_unscale[1] = floats_to_scaled_half(fl.data(), fl.size(), h16);
-            upload(L.sh_gu16, half, h16.data(), half);
+            upload_later(L.sh_gu16, half, h16.data(), half);
             L.sh_down16 = dev.buffer(half, Kind::device);
             shared_to_floats(kind, d.sh_down, E, SF, fl);
             L.sh_unscale[2] = floats_to_scaled_half(fl.data(), fl.size(), h16);
-            upload(L.sh_down16, 0, h16.data(), half);
+            upload_later(L.sh_down16, 0, h16.data(), half);
             if (!x16.handle) x16 = dev.buffer((uint64_t)max_tok * E * 2, Kind::device);
             if (d.SF > sh_width) {
                 for (Buffer *b : {&sh_h, &sh_a, &sh_o, &sh_g, &sh_s})
@@ -708,6 +824,9 @@ class Engine {
                 sh_width = d.SF;
             }
         }
+        // Callers may read the layer on a stream of their own next (gm_forward_decode_noalloc).
+        dev.begin();
+        dev.wait(submit());
         layers.push_back(L);
         return il;
     }
@@ -869,18 +988,19 @@ class Engine {
         explicit UnfusedPrefillScope(Engine *eng) : e(eng), was(eng->prefill_fused) { e->prefill_fused = false; }
         ~UnfusedPrefillScope() { e->prefill_fused = was; }
     };
-    // Reads and clears the give-up word of the persistent GEMMs: set when a down unit stopped waiting
-    // for its tile's gate/up rows (the call's outputs are then invalid).
-    bool take_gemm_error() {
-        if (!gemm_sched.handle) return false;
-        uint32_t w = 0;
-        check(gd_readback(dev.ctx, gemm_sched.handle, 4, 4, &w, kTimeoutMs), "gd_readback");
-        if (!w) return false;
+    // Clears the give-up word of the persistent GEMMs: set when a down unit stopped waiting for its
+    // tile's gate/up rows (the call's outputs are then invalid).
+    void clear_gemm_error() {
         const uint32_t zero = 0;
         upload(gemm_sched, 4, &zero, 4);
-        return true;
     }
-
+    // Clears the activation range flags: set when a fast-path kernel rounded an activation outside the
+    // binary16 range.
+    void clear_range_flag() {
+        const uint32_t zero = 0;
+        upload(range_flag, 0, &zero, 4);
+        upload(meta, kMetaRangeFlag * 4, &zero, 4);
+    }
 
     // MI355X decode path: router + rotation, routed gate/up, down + combine.
     void ffn_decode(uint32_t il, uint32_t n, uint32_t x_uav, uint32_t x_off, uint32_t out_uav, uint32_t out_off,
@@ -1190,38 +1310,31 @@ class Engine {
     void forward_stack(const uint32_t *list, uint32_t n_layers, uint32_t path, const float *x, uint32_t n, float *y) {
         if (n == 0 || n > max_tok) throw NativeError(-1, "token count exceeds max_tok");
         check_stack(list, n_layers);
-        upload(x_in, 0, x, (uint64_t)n * E * 4);
-        dev.begin();
-        stack(list, n_layers, path, n, x_in.uav, 0, x_in.uav, 0);
-        dev.wait(dev.submit());
-        if (path == GM_PATH_PREFILL && take_gemm_error()) {
-            UnfusedPrefillScope unfused{this};
-            upload(x_in, 0, x, (uint64_t)n * E * 4);
-            dev.begin();
-            stack(list, n_layers, path, n, x_in.uav, 0, x_in.uav, 0);
-            dev.wait(dev.submit());
-        }
-        if (fast_path(path) && take_range_flag()) {
-            upload(x_in, 0, x, (uint64_t)n * E * 4);
-            dev.begin();
-            stack(list, n_layers, GM_PATH_GENERIC, n, x_in.uav, 0, x_in.uav, 0);
-            dev.wait(dev.submit());
-        }
-        check(gd_readback(dev.ctx, x_in.handle, 0, n * E * 4, y, kTimeoutMs), "gd_readback");
+        const uint64_t bytes = (uint64_t)n * E * 4;
+        auto once = [&](uint32_t p) {
+            begin_upload(x_in, 0, x, bytes);
+            stack(list, n_layers, p, n, x_in.uav, 0, x_in.uav, 0);
+            return finish_download(x_in, y, bytes, fast_path(p));
+        };
+        run_checked(path, once);
     }
 
-    // Reads and clears the activation range flags; true when a fast-path kernel rounded an
-    // activation outside the binary16 range since the last call.
-    bool take_range_flag() {
-        uint32_t f = 0, g = 0;
-        check(gd_readback(dev.ctx, range_flag.handle, 0, 4, &f, kTimeoutMs), "gd_readback");
-        if (meta.handle) check(gd_readback(dev.ctx, meta.handle, kMetaRangeFlag * 4, 4, &g, kTimeoutMs), "gd_readback");
-        if (!f && !g) return false;
-        const uint32_t zero = 0;
-        upload(range_flag, 0, &zero, 4);
-        if (meta.handle) upload(meta, kMetaRangeFlag * 4, &zero, 4);
-        return true;
+    // One call through once(path), and again where its flags say that the outputs are not valid: after a
+    // give-up with two GEMM launches, after an activation outside the binary16 range on the generic path.
+    template <class Once>
+    void run_checked(uint32_t path, Once &&once) {
+        Flags f = once(path);
+        if (f.gemm_error) {
+            clear_gemm_error();
+            UnfusedPrefillScope unfused{this};
+            f = once(path);
+        }
+        if (f.range) {
+            clear_range_flag();
+            once(GM_PATH_GENERIC);
+        }
     }
+
     // The flag's table index for kernels of the fast paths (none on direct launches, whose
     // callers do not read it).
     uint32_t flag_uav() const { return direct ? 0u : range_flag.uav; }
@@ -1276,22 +1389,13 @@ class Engine {
 
     void forward(uint32_t il, uint32_t path, const float *x, uint32_t n, float *y) {
         if (n == 0 || n > max_tok) throw NativeError(-1, "token count exceeds max_tok");
-        upload(x_in, 0, x, (uint64_t)n * E * 4);
-        dev.begin();
-        ffn(path, il, n, x_in.uav, 0, out.uav, 0);
-        dev.wait(dev.submit());
-        if (path == GM_PATH_PREFILL && take_gemm_error()) {
-            UnfusedPrefillScope unfused{this};
-            dev.begin();
-            ffn(path, il, n, x_in.uav, 0, out.uav, 0);
-            dev.wait(dev.submit());
-        }
-        if (fast_path(path) && take_range_flag()) {
-            dev.begin();
-            ffn(GM_PATH_GENERIC, il, n, x_in.uav, 0, out.uav, 0);
-            dev.wait(dev.submit());
-        }
-        check(gd_readback(dev.ctx, out.handle, 0, n * E * 4, y, kTimeoutMs), "gd_readback");
+        const uint64_t bytes = (uint64_t)n * E * 4;
+        auto once = [&](uint32_t p) {
+            begin_upload(x_in, 0, x, bytes);
+            ffn(p, il, n, x_in.uav, 0, out.uav, 0);
+            return finish_download(out, y, bytes, fast_path(p));
+        };
+        run_checked(path, once);
     }
 };
 
@@ -1448,7 +1552,8 @@ extern "C" int gm_run_bracketed(gm_engine *g, uint32_t path, uint32_t batch, uin
                       &marks);
             }
             marks.push_back(e.dev.timestamp());
-            e.dev.wait(e.dev.submit());
+            if (last == calls && Engine::fast_path(path)) e.record_flags();
+            e.dev.wait(e.submit());
             std::vector<uint64_t> ticks(marks.size());
             const uint64_t freq = e.dev.timestamps(ticks.data(), (uint32_t)ticks.size());
             dev += (double)(ticks.back() - ticks.front()) * 1e3 / (double)freq;
@@ -1460,10 +1565,13 @@ extern "C" int gm_run_bracketed(gm_engine *g, uint32_t path, uint32_t batch, uin
         *wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         *device_ms = dev;
         if (bracket_us) *bracket_us = br_n ? br / (double)br_n : 0.0;
-        if (path == GM_PATH_PREFILL && e.take_gemm_error())
+        const Engine::Flags f = calls && Engine::fast_path(path) ? e.flags() : Engine::Flags{};
+        if (f.gemm_error) e.clear_gemm_error();
+        else if (f.range) e.clear_range_flag();
+        if (f.gemm_error)
             throw gyro::NativeError(-1, "a prefill GEMM unit gave up waiting for its tile's gate/up rows: the outputs of "
                                         "this run are invalid (gm_forward recomputes such calls with two GEMM launches)");
-        if (Engine::fast_path(path) && e.take_range_flag())
+        if (f.range)
             throw gyro::NativeError(-1, "an activation left the binary16 range on the prefill path: the outputs of this run "
                                         "are invalid (gm_forward recomputes such calls on GM_PATH_GENERIC)");
     });
@@ -1495,17 +1603,21 @@ extern "C" int gm_run_stack(gm_engine *g, uint32_t path, uint32_t batch, uint32_
                 e.stack(layer_list, n_layers, path, batch, e.tokens.uav, off, e.outputs.uav, off);
             }
             const uint32_t t_end = e.dev.timestamp();
-            e.dev.wait(e.dev.submit());
+            if (last == calls && Engine::fast_path(path)) e.record_flags();
+            e.dev.wait(e.submit());
             std::vector<uint64_t> ticks(t_end + 1);
             const uint64_t freq = e.dev.timestamps(ticks.data(), (uint32_t)ticks.size());
             dev += (double)(ticks[t_end] - ticks[t_start]) * 1e3 / (double)freq;
         }
         *wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         *device_ms = dev;
-        if (path == GM_PATH_PREFILL && e.take_gemm_error())
+        const Engine::Flags f = calls && Engine::fast_path(path) ? e.flags() : Engine::Flags{};
+        if (f.gemm_error) e.clear_gemm_error();
+        else if (f.range) e.clear_range_flag();
+        if (f.gemm_error)
             throw gyro::NativeError(-1, "a prefill GEMM unit gave up waiting for its tile's gate/up rows: the outputs of "
                                         "this run are invalid (gm_forward_stack recomputes such calls with two GEMM launches)");
-        if (Engine::fast_path(path) && e.take_range_flag())
+        if (f.range)
             throw gyro::NativeError(-1, "an activation left the binary16 range on the prefill path: the outputs of this run "
                                         "are invalid (gm_forward_stack recomputes such calls on GM_PATH_GENERIC)");
     });
@@ -1522,8 +1634,6 @@ extern "C" int gm_read_outputs(gm_engine *g, float *y, uint32_t n_total) {
     return guarded(g, [&] {
         Engine &e = g->e;
         if (n_total > e.n_tokens) throw gyro::NativeError(-1, "more outputs than tokens");
-        gyro::check(gd_readback(e.dev.ctx, e.outputs.handle, 0, (uint32_t)((uint64_t)n_total * e.E * 4), y,
-                                gyro::kTimeoutMs),
-                    "gd_readback");
+        e.download(e.outputs, y, (uint64_t)n_total * e.E * 4);
     });
 }
