@@ -64,3 +64,41 @@ __device__ __forceinline__ void gd_fwht128_x16(float (&v)[16], uint32_t l8) {
         v[j] = (l8 & 4u) ? dn4 - v[j] : v[j] + up4;
     }
 }
+
+// The same held by a 16-lane row, 8 consecutive values per lane: lane l16 of the row holds elements
+// 8 l16 .. 8 l16 + 7 in v (the widths in the same order: 1..4 in registers, 8..64 across lanes).
+__device__ __forceinline__ void gd_fwht128_x8(float (&v)[8], uint32_t l16) {
+    // Widths 1..4: element bits 0..2 are the register index bits.
+#pragma unroll
+    for (int w = 1; w < 8; w <<= 1)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (!(j & w)) {
+                const float lo = v[j], hi = v[j + w];
+                v[j] = lo + hi;
+                v[j + w] = lo - hi;
+            }
+    // Widths 8, 16, 32, 64: partners are lanes l16 ^ 1, ^ 2, ^ 4, ^ 8 of the 16-lane row.
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float p1 = gd_dpp_f<0xB1>(v[j]);  // quad_perm [1,0,3,2]
+        v[j] = (l16 & 1u) ? p1 - v[j] : v[j] + p1;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float p2 = gd_dpp_f<0x4E>(v[j]);  // quad_perm [2,3,0,1]
+        v[j] = (l16 & 2u) ? p2 - v[j] : v[j] + p2;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float up4 = gd_dpp_f<0x104>(v[j]);  // row_shl:4, lane + 4
+        const float dn4 = gd_dpp_f<0x114>(v[j]);  // row_shr:4, lane - 4
+        v[j] = (l16 & 4u) ? dn4 - v[j] : v[j] + up4;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float up8 = gd_dpp_f<0x108>(v[j]);  // row_shl:8, lane + 8
+        const float dn8 = gd_dpp_f<0x118>(v[j]);  // row_shr:8, lane - 8
+        v[j] = (l16 & 8u) ? dn8 - v[j] : v[j] + up8;
+    }
+}

@@ -186,6 +186,57 @@ __device__ __forceinline__ float tq2_block_dot_halves(const uint32_t q[8], const
     return acc0 + acc1;
 }
 
+// One stream word of a block in phases, for software pipelining: tq2_word_states gives the two state
+// pairs of word i (of the block's nine words d as tq2_unpack takes them), tq2_state_gather issues the two
+// codebook reads of state j of the four, tq2_state_fma adds their products with the state's four
+// activations x to acc0 and acc1. Words 0 .. 7 in turn give tq2_block_dot's sums bit for bit.
+__device__ __forceinline__ void tq2_word_states(const uint32_t (&d)[9], bool odd_half, int i, uint32_t (&p)[2]) {
+    const int prev = (i + 7) & 7;
+    const uint32_t q = odd_half ? d[i + 1] : __builtin_amdgcn_alignbyte(d[i + 1], d[i], 2);
+    const uint32_t qp = odd_half ? d[prev + 1] : d[prev + 1] << 16;  // its top byte is all that is read
+    p[0] = tq2_pair01(q, qp);
+    p[1] = tq2_pair23(q);
+}
+__device__ __forceinline__ void tq2_state_gather(const uint32_t (&p)[2], int j, const uint32_t *book, uint32_t (&raw)[2]) {
+    uint32_t a0, a1;
+    cb_addr(j & 1 ? __builtin_amdgcn_ubfe(p[j >> 1], 16, 15) : p[j >> 1] & 0x7fffu, a0, a1);
+    raw[0] = lds_word(book, a0);
+    raw[1] = lds_word(book, a1);
+}
+__device__ __forceinline__ void tq2_state_fma(const uint32_t (&raw)[2], const float *x, float &acc0, float &acc1) {
+    acc0 = fma_lo(raw[0], x[0], acc0);
+    acc1 = fma_hi(raw[0], x[1], acc1);
+    acc0 = fma_lo(raw[1], x[2], acc0);
+    acc1 = fma_hi(raw[1], x[3], acc1);
+}
+
+// tq2_half_dot of a half block held as the five words w that span its stream words (as the block's nine
+// words d[4 half .. 4 half + 4]) and qp, whose top byte is the stream byte before the half's first.
+__device__ __forceinline__ float tq2_half_words_dot(const uint32_t (&w)[5], bool odd_half, uint32_t qp,
+                                                    const uint32_t *book, const float (&x)[64]) {
+    float acc0 = 0.f, acc1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t q = odd_half ? w[i + 1] : __builtin_amdgcn_alignbyte(w[i + 1], w[i], 2);
+        const uint32_t p01 = tq2_pair01(q, qp), p23 = tq2_pair23(q);
+        qp = q;
+        const uint32_t s[4] = {p01 & 0x7fffu, __builtin_amdgcn_ubfe(p01, 16, 15), p23 & 0x7fffu,
+                               __builtin_amdgcn_ubfe(p23, 16, 15)};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t a0, a1;
+            cb_addr(s[j], a0, a1);
+            const uint32_t w0 = lds_word(book, a0), w1 = lds_word(book, a1);
+            const float *xs = x + (i * 4 + j) * 4;
+            acc0 = fma_lo(w0, xs[0], acc0);
+            acc1 = fma_hi(w0, xs[1], acc1);
+            acc0 = fma_lo(w1, xs[2], acc0);
+            acc1 = fma_hi(w1, xs[3], acc1);
+        }
+    }
+    return acc0 + acc1;
+}
+
 // The 9 words from the 4-byte-aligned start of the 34-byte block at byte `off` (even) of `base`.
 __device__ __forceinline__ void tq2_load_block(const uint8_t *base, uint64_t off, uint32_t d[9]) {
     gd_guint *w = gd_global(reinterpret_cast<const uint32_t *>(base + (off & ~uint64_t(3))));

@@ -103,39 +103,7 @@ GD_PIPELINE_NAMED(moe_decode_down, 512) {
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int c = 0; c < 4; ++c) v[4 * j + c] *= gd_bits_f32(s4[j][c]);
-        // Widths 1..4: element bits 0..2 are the register index bits.
-#pragma unroll
-        for (int w = 1; w < 8; w <<= 1)
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (!(j & w)) {
-                    const float lo = v[j], hi = v[j + w];
-                    v[j] = lo + hi;
-                    v[j + w] = lo - hi;
-                }
-        // Widths 8, 16, 32, 64: partners are lanes l16 ^ 1, ^ 2, ^ 4, ^ 8 of the 16-lane row.
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float p1 = gd_dpp_f<0xB1>(v[j]);  // quad_perm [1,0,3,2]
-            v[j] = (l16 & 1u) ? p1 - v[j] : v[j] + p1;
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float p2 = gd_dpp_f<0x4E>(v[j]);  // quad_perm [2,3,0,1]
-            v[j] = (l16 & 2u) ? p2 - v[j] : v[j] + p2;
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float up4 = gd_dpp_f<0x104>(v[j]);  // row_shl:4, lane + 4
-            const float dn4 = gd_dpp_f<0x114>(v[j]);  // row_shr:4, lane - 4
-            v[j] = (l16 & 4u) ? dn4 - v[j] : v[j] + up4;
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float up8 = gd_dpp_f<0x108>(v[j]);  // row_shl:8, lane + 8
-            const float dn8 = gd_dpp_f<0x118>(v[j]);  // row_shr:8, lane - 8
-            v[j] = (l16 & 8u) ? dn8 - v[j] : v[j] + up8;
-        }
+        gd_fwht128_x8(v, l16);
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] *= GD_INV_SQRT128;
     }

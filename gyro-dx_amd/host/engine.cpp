@@ -951,9 +951,9 @@ class Engine {
         dispatch("moe_combine", {down.uav, 0, weights.uav, 0, out_uav, out_off, U, E, sh, 0, shg, 0}, (E + 255) / 256, n);
     }
 
-    // Routed experts: uniform TQ2_T layers take moe_decode_gu (one token) or moe_decode_gu_b (2-8)
-    // and moe_decode_down (E 1024 or 2048,
-    // F 512, top-8) or moe_decode_gu_g and moe_decode_down_g / _gl (E a multiple of 256 up to 4096,
+    // Routed experts: uniform TQ2_T layers take moe_decode_gu and moe_decode_down (one token) or
+    // moe_decode_gu_r2 / _r4 and moe_decode_down_r2 / _r4 (batches) at E 1024 or 2048,
+    // F 512, top-8, or moe_decode_gu_g and moe_decode_down_g / _gl (E a multiple of 256 up to 4096,
     // F a multiple of 128 up to 1024, top-1..16); other layers the type-generic kernels (_x for E
     // a multiple of 1024, F 512, top-8; _xg otherwise).
     // Shared expert: a bf16 one of width <= 1024 (a multiple of 256) on E <= 2048 at the _x shapes
@@ -972,6 +972,18 @@ class Engine {
     // Uniform TQ2_T layers take moe_decode_gu / moe_decode_down at their compile-time shape
     // (hidden 1024 or 2048, F 512, top-8), moe_decode_gu_g / moe_decode_down_g(l) otherwise.
     bool decode_tuned_tq2() const { return E % 1024 == 0 && F == 512 && U == 8 && parts <= 2; }
+    // Blocks a lane of the batch kernels decodes at the tuned shape: 4 or 2, where the groups (E n / 32 and
+    // E n / 16) fill at least 7/8 of whole rounds of 256 (2, 4 and 6 to 8 tokens at hidden 2048), else 0:
+    // moe_decode_gu_b and moe_decode_down, whose 2,048 smaller groups balance better.
+    // Four layers replayed, us without and with: hidden 2048, 2 tokens 81 -> 76, 4 112 -> 105, 6 145 -> 133,
+    // 8 176 -> 154; forced at 3 tokens 96 -> 100, at 5 126 -> 147; hidden 1024, 4 tokens 82 -> 77, 8 114 -> 107.
+    uint32_t decode_blocks_per_lane(uint32_t n) const {
+        for (uint32_t r : {4u, 2u}) {
+            const uint32_t groups = E * n / (8 * r), rounds = (groups + 255) / 256;
+            if (8 * groups >= 7 * 256 * rounds) return r;
+        }
+        return 0;
+    }
     uint32_t cus_or(uint32_t fallback) const { return cus ? cus : fallback; }
     bool decode_fused_shared(const Layer &L) const {
         return L.SF && L.sh_kind == GM_SHARED_BF16 && decode_generic_tuned() && L.SF <= 1024 && L.SF % 256 == 0 &&
@@ -1043,18 +1055,28 @@ class Engine {
         }
         if (!generic || !decode_generic_tuned()) {
             if (!generic && decode_tuned_tq2()) {
-                // One token: the build that holds a block's activations in registers at once;
-                // more: the half-block build, which lets four groups share a compute unit.
-                dispatch_maybe_timed(bracket == 2, marks, n == 1 ? "moe_decode_gu" : "moe_decode_gu_b",
-                                     {B.logits, B.logits_off, NE, U, bits(L.scale), B.ids, B.ids_off, B.weights, B.weights_off, B.xh,
-                                      B.xh_off, base_lo, base_hi, slot_stride, L.gate_bytes, codebook.srv, B.gu, B.gu_off, E, F, n},
-                                     F / 64, 2 * parts, n * U);
-                dispatch_maybe_timed(bracket == 3, marks, "moe_decode_down",
-                                     {B.gu, B.gu_off, B.ids, B.ids_off, B.weights, B.weights_off, base_lo, base_hi, slot_stride,
-                                      2 * L.gate_bytes, codebook.srv, L.has_down_signs ? L.signs.srv : kNone, E, out_uav,
-                                      out_off, E, F, U, n, parts, NE, st.res_uav != kNone ? 1u : 0u, st.res_uav,
-                                      st.res_off},
-                                     E / 8, n);
+                // One token: the build that holds a block's activations in registers at once. Batches:
+                // several blocks per lane against one register copy of the activations, or one block
+                // per lane, four groups per CU.
+                const std::initializer_list<uint32_t> gu = {B.logits, B.logits_off, NE, U, bits(L.scale), B.ids, B.ids_off, B.weights,
+                                                  B.weights_off, B.xh, B.xh_off, base_lo, base_hi, slot_stride, L.gate_bytes,
+                                                  codebook.srv, B.gu, B.gu_off, E, F, n};
+                const std::initializer_list<uint32_t> dn = {B.gu, B.gu_off, B.ids, B.ids_off, B.weights, B.weights_off, base_lo, base_hi,
+                                                  slot_stride, 2 * L.gate_bytes, codebook.srv,
+                                                  L.has_down_signs ? L.signs.srv : kNone, E, out_uav, out_off, E, F, U, n, parts,
+                                                  NE, st.res_uav != kNone ? 1u : 0u, st.res_uav, st.res_off};
+                const uint32_t r = n == 1 ? 0u : decode_blocks_per_lane(n);
+                if (r) {
+                    const uint32_t rows = 8 * (64 / (E / 128)) * r / 2;  // gate/up rows of a group
+                    dispatch_maybe_timed(bracket == 2, marks, r == 4 ? "moe_decode_gu_r4" : "moe_decode_gu_r2", gu,
+                                         F / rows, 1, n * U);
+                    dispatch_maybe_timed(bracket == 3, marks, r == 4 ? "moe_decode_down_r4" : "moe_decode_down_r2", dn,
+                                         E / (8 * r), n);
+                    return;
+                }
+                dispatch_maybe_timed(bracket == 2, marks, n == 1 ? "moe_decode_gu" : "moe_decode_gu_b", gu, F / 64, 2 * parts,
+                                     n * U);
+                dispatch_maybe_timed(bracket == 3, marks, "moe_decode_down", dn, E / 8, n);
                 return;
             }
             // Other shapes: runs of RPG (token, slot, row) rows per gate/up group (at most 1024
