@@ -22,11 +22,20 @@
 // 4 weights_uav 5 weights_off 6 base_lo 7 base_hi 8 slot_stride 9 down_off 10 codebook_srv
 // 11 signs_srv (0xffffffff: none) 12 signs_off 13 out_uav (or its address in 58, 59) 14 out_off 15 E 16 F 17 n_used
 // 18 n_tok 19 R 20 n_expert 21 residual 22 res_uav 23 res_off (24 xtab_srv: the generic form).
+// Builds with DG_SHARED (moe_decode_down_gs, _xgs) add the shared expert's gated down rows,
+// sigmoid(g[t]) * (W_sd[r] . a[t]) with a and g from moe_router_s: 25 row format (0 bf16, 1 Q8_0) 26 a_uav
+// 27 a_off (fp32 [n][SF]) 28 g_uav 29 g_off 30 w_srv 31 row bytes 32 SF (a multiple of 64 up to 1024);
+// R <= 16. A wave takes rows w and w + 8 of the group: their loads (at most 16 bytes x 2 a lane and row) go
+// out before the routed blocks', and the products run while those are in flight, so the launch of
+// moe_decode_shared_down and its gap go. Measured, four
+// layers replayed at hidden 2560, F 640, top-10, Q8_0 of width 640: 1 token 116 -> 102 us, 2 tokens
+// 166 -> 151, 8 tokens 497 -> 476; GGUF 148 at 2 tokens 202 -> 188; bf16 of width 1024 at 2 tokens 169 -> 155.
 // Requires TQ2_T experts (any types in the generic form), F a multiple of 128 up to 1024,
 // 1 <= n_used <= 16, n_used F / 128 <= DG_MAX_ABLK, n_used F / 64 ceil(R / 2) <= 512 DG_ITEMS
 // and R n_used <= 512 (the host checks).
 #include "gyro_fast.h"
 #include "fwht.h"
+#include "shared_rows.h"
 
 #ifndef DG_MAX_ABLK
 #define DG_MAX_ABLK 64  // rotated input blocks (slots x F / 128) in LDS
@@ -34,6 +43,9 @@
 #endif
 #ifndef DG_GENERIC
 #define DG_GENERIC 0  // 1: any Gyro type per expert, rows from the expert table
+#endif
+#ifndef DG_SHARED
+#define DG_SHARED 0  // 1: the shared expert's down rows too
 #endif
 // Words loaded per block: TQ2_T's 34 bytes, or the widest type's 58 (whole words from the
 // block's first byte rounded down to a word; the arena's slack covers reads past the last row).
@@ -53,6 +65,9 @@ DG_DEFINE(DG_PIPELINE, 512) {
     __shared__ float actr[DG_MAX_ABLK * DG_BLOCK_STRIDE];
     __shared__ float dred[2 * DG_ITEMS * 512];  // half dots by (slot, row, block, half)
     __shared__ float sw[DG_MAX_U];
+#if DG_SHARED
+    __shared__ float shs[16];  // W_sd[r0 + i] . a[t]
+#endif
 #if DG_GENERIC
     __shared__ gd_u32x4 xdesc[DG_MAX_EXPERTS];  // per expert {down lo, down hi, types, pad}
 #endif
@@ -116,6 +131,46 @@ DG_DEFINE(DG_PIPELINE, 512) {
         svv[ps][0] = S[0];
         svv[ps][1] = S[1];
     }
+#if DG_SHARED
+    // Rows `wave` and `wave` + 8 of the group (a wave past the last repeats it), columns 16 lane (Q8_0) or
+    // 8 lane and 512 + 8 lane (bf16); lanes past the last column read it again and multiply zeros.
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), SF = a.c[32];
+    const bool q8 = a.c[25] != 0u;  // uniform
+    const float sg_dot = gd_bits_f32(gd_global(gd_buf<const uint32_t>(a, a.c[28]) + a.c[29])[t]);
+    gd_u32x4 shw[2][2], shx[4];
+    uint32_t shd[2] = {0u, 0u};
+    bool shin[2];
+    {
+        const uint32_t *A = gd_buf<const uint32_t>(a, a.c[26]) + a.c[27] + (size_t)t * SF;
+        const uint8_t *W = gd_buf<const uint8_t>(a, a.c[30]);
+        const uint8_t *row[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) row[i] = W + (size_t)(r0 + min(wave + 8u * i, R - 1u)) * a.c[31];
+        if (q8) {
+            const uint32_t c = 16u * lane, col = c < SF ? c : SF - 16u;
+            shin[0] = c < SF;
+            shin[1] = false;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                shw[i][0] = *gd_global4(reinterpret_cast<const uint32_t *>(row[i] + col));
+                shw[i][1] = shw[i][0];
+                shd[i] = *(const __attribute__((address_space(1))) uint16_t *)(uintptr_t)(row[i] + SF + (col / 32u) * 2u);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) shx[j] = *gd_global4(A + col + 4u * j);
+        } else {
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const uint32_t c = 8u * (64u * m + lane), col = c < SF ? c : SF - 8u;
+                shin[m] = c < SF;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) shw[i][m] = *gd_global4(reinterpret_cast<const uint32_t *>(row[i] + 2u * col));
+#pragma unroll
+                for (int j = 0; j < 2; ++j) shx[2 * m + j] = *gd_global4(A + col + 4u * j);
+            }
+        }
+    }
+#endif
 #if DG_GENERIC
     if (tid < NE) xdesc[tid] = xdv;
     __syncthreads();
@@ -205,6 +260,31 @@ DG_DEFINE(DG_PIPELINE, 512) {
         dst[0] = make_float4(v[0], v[1], v[2], v[3]);
         dst[1] = make_float4(v[4], v[5], v[6], v[7]);
     }
+#if DG_SHARED
+    // The sums in shr_dots' order: a lane's columns, then the wave.
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        float p = 0.f;
+        if (q8) {
+            float v[16], d = 0.f;
+            shr_values<SHR_Q8>(shw[i][0], gd_half(shd[i]), v);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) d += v[j] * gd_bits_f32(shx[j / 4][j % 4]);
+            p += shin[0] ? d : 0.f;
+        } else {
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                float v[8], d = 0.f;
+                shr_values<SHR_BF16>(shw[i][m], 1.f, v);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) d += v[j] * gd_bits_f32(shx[2 * m + j / 4][j % 4]);
+                p += shin[m] ? d : 0.f;
+            }
+        }
+        p = gd_wave_sum_dpp(p);
+        if (lane == 0u && wave + 8u * i < R) shs[wave + 8u * i] = p;
+    }
+#endif
     __syncthreads();
 
     // Item dots: the half's 64 activations from LDS once, then that half of both rows' blocks;
@@ -276,7 +356,12 @@ DG_DEFINE(DG_PIPELINE, 512) {
         }
         if (k16 == U - 1u) {
             const uint32_t o = t * E + r0 + row;
+#if DG_SHARED
+            const float sh = gd_sigmoid_accurate(sg_dot) * shs[row];
+            acc = (residual ? gd_bits_f32(resv) + sh : sh) + acc;
+#else
             if (residual) acc = (row < 32u ? gd_bits_f32(resv) : RES[o]) + acc;
+#endif
             OUT[o] = acc;
         }
     }

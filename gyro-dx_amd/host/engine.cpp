@@ -959,7 +959,7 @@ class Engine {
     // Shared expert: a bf16 one of width <= 1024 (a multiple of 256) on E <= 2048 at the _x shapes
     // runs fused into moe_router and moe_decode_down_x; any other (bf16, Q8_0 or fp32, any width
     // a multiple of 64) runs its gate and up rows in the router's launch (moe_router_s) and its down rows
-    // in moe_decode_shared_down, whose output sigmoid(g . x) * W_d (silu(W_g x) * W_u x) enters the
+    // in the routed down kernel (decode_folds_shared_down) or in moe_decode_shared_down, whose output sigmoid(g . x) * W_d (silu(W_g x) * W_u x) enters the
     // routed down kernel as its residual input.
     bool decode_supported(const Layer &L, uint32_t n) const {
         if (NE > 256 || n > 8 || E > 4096) return false;
@@ -983,6 +983,19 @@ class Engine {
             if (8 * groups >= 7 * 256 * rounds) return r;
         }
         return 0;
+    }
+    // Output rows of a moe_decode_down_g group: about one group per CU for a token, within its item and sum limits.
+    uint32_t decode_down_rows() const {
+        uint32_t R = std::max(1u, E / cus_or(256));
+        while (R > 1 && (E % R || U * (F / 128) * 2 * ((R + 1) / 2) > 1024 || R * U > 512)) --R;
+        return R;
+    }
+    // Whether moe_decode_down_gs / _xgs takes the layer's shared down rows along (no moe_decode_shared_down):
+    // the shapes of the _g kernels whose groups keep one per CU (not _gl), at most two rows a wave, and rows
+    // of one 16-byte load (Q8_0) or two (bf16) a lane, held in registers beside the routed blocks.
+    bool decode_folds_shared_down(const Layer &L) const {
+        if (!L.SF || decode_fused_shared(L) || L.SF > 1024 || L.sh_kind == GM_SHARED_F32 || decode_down_rows() > 16) return false;
+        return decode_generic_types(L) ? !decode_generic_tuned() : !decode_tuned_tq2() && U * (F / 128) <= 64;
     }
     uint32_t cus_or(uint32_t fallback) const { return cus ? cus : fallback; }
     bool decode_fused_shared(const Layer &L) const {
@@ -1027,10 +1040,11 @@ class Engine {
         const bool fused_sh = decode_fused_shared(L);
         const uint32_t rsf = fused_sh ? L.SF : 0u;  // shared rows computed inside moe_router
         const uint32_t base_lo = (uint32_t)L.base, base_hi = (uint32_t)(L.base >> 32);
-        const bool generic = decode_generic_types(L);
+        const bool generic = decode_generic_types(L), folded = decode_folds_shared_down(L);
         if (L.SF && !fused_sh) {
-            // The shared expert's SwiGLU rows and gate dots in the router's launch, its gated output (plus
-            // a stack's stream) in a launch of its own: the residual input of the down kernel.
+            // The shared expert's SwiGLU rows and gate dots in the router's launch, its gated down rows in the
+            // routed down kernel (folded) or, plus a stack's stream, in a launch of their own: the residual
+            // input of the down kernel.
             const SharedBufs &S = B.shared;
             dispatch_maybe_timed(bracket == 1, marks, "moe_router_s",
                                  {x_uav, x_off, E, n, L.router.srv, 0, NE, E, L.has_bias ? L.bias.srv : kNone, 0,
@@ -1038,12 +1052,14 @@ class Engine {
                                   0, 0, 0, 0, L.SF, L.sh_gu.srv, S.a, L.sh_gate.srv, S.g, L.sh_row_e, L.sh_kind, S.a_off,
                                   S.g_off},
                                  NE + E / 128 + L.SF / 4 + 1);
-            dispatch("moe_decode_shared_down",
-                     {S.a, S.a_off, S.g, S.g_off, L.sh_down.srv, L.sh_row_f, L.sh_kind, L.SF, E, n, S.s, S.s_off,
-                      st.res_uav != kNone ? 1u : 0u, st.res_uav != kNone ? st.res_uav : 0u, st.res_off},
-                     (E + 7) / 8);
-            st.res_uav = S.s;
-            st.res_off = S.s_off;
+            if (!folded) {
+                dispatch("moe_decode_shared_down",
+                         {S.a, S.a_off, S.g, S.g_off, L.sh_down.srv, L.sh_row_f, L.sh_kind, L.SF, E, n, S.s, S.s_off,
+                          st.res_uav != kNone ? 1u : 0u, st.res_uav != kNone ? st.res_uav : 0u, st.res_off},
+                         (E + 7) / 8);
+                st.res_uav = S.s;
+                st.res_off = S.s_off;
+            }
         } else {
             dispatch_maybe_timed(bracket == 1, marks, "moe_router",
                                  {x_uav, x_off, E, n, L.router.srv, 0, NE, E, L.has_bias ? L.bias.srv : kNone, 0,
@@ -1086,21 +1102,25 @@ class Engine {
             // form (_xg: rows through the expert table, each expert's types).
             const uint32_t nb = E / 128, total = n * U * F, target = cus_or(256);
             const uint32_t rpg = std::max(1u, std::min({(total + target - 1) / target, F, 1024u / nb}));
-            uint32_t R = std::max(1u, E / target);
-            while (R > 1 && (E % R || U * (F / 128) * 2 * ((R + 1) / 2) > 1024 || R * U > 512)) --R;
+            const uint32_t R = decode_down_rows();
             const uint32_t xt = generic ? L.xtab.srv : 0u;
             dispatch_maybe_timed(bracket == 2, marks, generic ? "moe_decode_gu_xg" : "moe_decode_gu_g",
                                  {B.logits, B.logits_off, NE, U, bits(L.scale), B.ids, B.ids_off, B.weights, B.weights_off, B.xh,
                                   B.xh_off, generic ? 0u : base_lo, generic ? 0u : base_hi, generic ? 0u : slot_stride,
                                   generic ? 0u : L.gate_bytes, codebook.srv, B.gu, B.gu_off, E, F, n, rpg, xt},
                                  (total + rpg - 1) / rpg);
-            const char *down = generic ? "moe_decode_down_xg"
-                                       : (U * (F / 128) <= 64 ? "moe_decode_down_g" : "moe_decode_down_gl");
+            const char *down = generic ? (folded ? "moe_decode_down_xgs" : "moe_decode_down_xg")
+                               : folded ? "moe_decode_down_gs"
+                                        : (U * (F / 128) <= 64 ? "moe_decode_down_g" : "moe_decode_down_gl");
+            const SharedBufs &S = B.shared;
             dispatch_maybe_timed(bracket == 3, marks, down,
                                  {B.gu, B.gu_off, B.ids, B.ids_off, B.weights, B.weights_off, generic ? 0u : base_lo,
                                   generic ? 0u : base_hi, generic ? 0u : slot_stride, generic ? 0u : 2 * L.gate_bytes,
                                   codebook.srv, L.has_down_signs ? L.signs.srv : kNone, E, out_uav, out_off, E, F, U, n, R, NE,
-                                  st.res_uav != kNone ? 1u : 0u, st.res_uav, st.res_off, xt},
+                                  st.res_uav != kNone ? 1u : 0u, st.res_uav, st.res_off, xt,
+                                  folded && L.sh_kind == GM_SHARED_Q8_0 ? 1u : 0u, folded ? S.a : 0u, folded ? S.a_off : 0u,
+                                  folded ? S.g : 0u, folded ? S.g_off : 0u, folded ? L.sh_down.srv : 0u,
+                                  folded ? L.sh_row_f : 0u, folded ? L.SF : 0u},
                                  E / R, n);
             return;
         }
