@@ -210,6 +210,45 @@ __device__ __forceinline__ void tq2_state_fma(const uint32_t (&raw)[2], const fl
     acc1 = fma_hi(raw[1], x[3], acc1);
 }
 
+// Unscaled dots of R blocks (nine words each, all of one start parity) with the same 128 activations (LDS, the
+// x33 layout), acc0[i] + acc1[i] in tq2_block_dot's order: half the activations go into registers at a
+// time and serve all R blocks. At most 128 VGPRs at R = 4.
+template <int R>
+__device__ __forceinline__ void tq2_blocks_dot(const uint32_t (&d)[R][9], bool odd, const uint32_t *book,
+                                               const uint4 *xb, float (&acc0)[R], float (&acc1)[R]) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) acc0[i] = acc1[i] = 0.f;
+    // Steps of one stream word each, in the order (half, block, word): the codebook reads of step s + 1
+    // are issued between the products of step s, state by state, with fences that hold the order.
+    uint32_t raw[2][4][2], pr[2];
+    tq2_word_states(d[0], odd, 0, pr);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tq2_state_gather(pr, j, book, raw[0][j]);
+    float x[64];
+#pragma unroll
+    for (int s = 0; s < 8 * R; ++s) {
+        const int h = s / (4 * R), i = (s / 4) % R, ii = s % 4, n = s + 1;
+        if (s % (4 * R) == 0) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const uint4 v = xb[16 * h + j];
+                x[4 * j] = gd_bits_f32(v.x);
+                x[4 * j + 1] = gd_bits_f32(v.y);
+                x[4 * j + 2] = gd_bits_f32(v.z);
+                x[4 * j + 3] = gd_bits_f32(v.w);
+            }
+        }
+        if (n < 8 * R) tq2_word_states(d[(n / 4) % R], odd, 4 * (n / (4 * R)) + n % 4, pr);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (n < 8 * R) tq2_state_gather(pr, j, book, raw[n & 1][j]);
+            __builtin_amdgcn_sched_barrier(0);
+            tq2_state_fma(raw[s & 1][j], x + 16 * ii + 4 * j, acc0[i], acc1[i]);
+            asm volatile("" : "+v"(acc0[i]), "+v"(acc1[i]));  // the products stay in their step
+        }
+    }
+}
+
 // tq2_half_dot of a half block held as the five words w that span its stream words (as the block's nine
 // words d[4 half .. 4 half + 4]) and qp, whose top byte is the stream byte before the half's first.
 __device__ __forceinline__ float tq2_half_words_dot(const uint32_t (&w)[5], bool odd_half, uint32_t qp,

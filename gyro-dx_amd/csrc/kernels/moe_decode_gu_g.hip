@@ -16,6 +16,11 @@
 //    src/kernels.zig:161-199); each row's gate and up sums in block order through LDS.
 //  - act[(t n_used + k) F + f] = silu(g) * u.
 // Expert e's rows are at base + e * slot_stride (+ proj_bytes for up): no table lookup.
+// Batch builds (GG_BATCH: moe_decode_gu_gb, moe_decode_gu_xgb): the same runs, items and sums in at most 128
+// VGPRs, so that two groups share a CU (sixteen waves against eight) and one routes, stages or waits for
+// its blocks while the other decodes: half of the activations in registers at a time (TQ2_T), or
+// read from LDS step by step (other types). Measured at hidden 2560, F 640,
+// top-10, four layers replayed: 3 tokens 198 -> 166 us, 8 tokens 412 -> 357, 8 tokens of GGUF 148 547 -> 486.
 // Grid: ceil(n_tok n_used F / RPG) groups; 512 threads.
 // Constants: 0 logits_uav 1 logits_off 2 n_expert 3 n_used 4 scale (fp32 bits) 5 ids_uav
 // 6 ids_off 7 weights_uav 8 weights_off 9 xh_uav (fp32 [n_tok][E]) 10 xh_off (words) 11 base_lo 12 base_hi
@@ -35,10 +40,17 @@
 #define GG_PIPELINE moe_decode_gu_g
 #define GG_GENERIC 0     // 1: any Gyro type per expert and projection, rows from the expert table
 #endif
+#ifndef GG_BATCH
+#define GG_BATCH 0
+#endif
 // Words loaded per block: TQ2_T's 34 bytes, or the widest type's 58 (whole words from the
 // block's first byte rounded down to a word; the arena's slack covers reads past the last row).
 #define GG_WORDS (GG_GENERIC ? 15 : 9)
-#define GG_DEFINE(NAME, WG) GD_PIPELINE_NAMED(NAME, WG)  // expands NAME before it is named
+#if GG_BATCH
+#define GG_DEFINE(NAME, WG) GD_PIPELINE_NAMED_OCC(NAME, WG, 4)  // expands NAME before it is named
+#else
+#define GG_DEFINE(NAME, WG) GD_PIPELINE_NAMED(NAME, WG)
+#endif
 
 // Selection rounds 0 .. need of one token (uniform per wave): the ids of ranks ka and kb; when
 // `writer`, every round and the token's ids and renormalised weights (rf_weights) stored by
@@ -93,7 +105,8 @@ GG_DEFINE(GG_PIPELINE, 512) {
 #if GG_GENERIC
     __shared__ gd_u32x4 xdesc[2 * 256];  // the expert table: {gate, up}, {down, types, pad} per expert
 #endif
-    __shared__ uint4 xh4[2][4096 / 4];  // the run's (up to) two tokens' rotated fp32 inputs
+    // The run's (up to) two tokens' rotated fp32 inputs; the batch builds read blocks at constant offsets.
+    __shared__ uint4 xh4[2][GG_BATCH ? 32 * 33 : 32 * 32];
     __shared__ float gred[2 * GG_ITEMS * 512];  // (row, projection) block dots
     __shared__ float gsum[2 * GG_MAX_RPG];
     __shared__ uint32_t sid[2];  // experts of the run's first and second slot
@@ -120,7 +133,7 @@ GG_DEFINE(GG_PIPELINE, 512) {
     for (uint32_t q = tid; q < (t1 != t0 ? 2u : 1u) * (E / 4u); q += 512u) {  // uint4 chunks
         const uint32_t ti = q / (E / 4u), c16 = q - ti * (E / 4u);
         const gd_u32x4 v = gd_global4(XH + (size_t)(ti ? t1 : t0) * E)[c16];
-        xh4[ti][x32_stage_index(c16 >> 5, c16 & 31u)] = make_uint4(v[0], v[1], v[2], v[3]);
+        xh4[ti][GG_BATCH ? x33_stage_index(c16 >> 5, c16 & 31u) : x32_stage_index(c16 >> 5, c16 & 31u)] = make_uint4(v[0], v[1], v[2], v[3]);
     }
 
     // Routing.
@@ -191,8 +204,16 @@ GG_DEFINE(GG_PIPELINE, 512) {
         if (j < n_items) {
             const uint32_t rr = j / nb, b = j - rr * nb;
             const uint32_t ti = (row0 + rr) / UF != t0 ? 1u : 0u;
+#if GG_BATCH && GG_GENERIC
+            const float *xf = reinterpret_cast<const float *>(xh4[ti] + b * 33u);
+#elif !GG_BATCH
             float xf[128];
             x32_from_lds(xh4[ti], b, xf);
+#endif
+#if GG_BATCH && !GG_GENERIC
+            float acc0[2], acc1[2];
+            tq2_blocks_dot<2>(dw[s], odd[s][0], book, xh4[ti] + b * 33u, acc0, acc1);
+#endif
 #pragma unroll
             for (int p = 0; p < 2; ++p) {
                 float v = 0.f;
@@ -206,6 +227,8 @@ GG_DEFINE(GG_PIPELINE, 512) {
     }
                 GYRO_TYPE_SWITCH(ty[s][p], GG_CASE)
 #undef GG_CASE
+#elif GG_BATCH
+                v = gd_half(odd[s][0] ? dw[s][p][0] >> 16 : dw[s][p][0] & 0xffffu) * (acc0[p] + acc1[p]);
 #else
                 float sc;
                 uint32_t q[8];

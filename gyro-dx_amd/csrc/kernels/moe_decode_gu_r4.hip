@@ -101,37 +101,7 @@ GU_DEFINE(GU_PIPELINE, 512) {
     const uint4 *xb = xall + b * 33u;
     const bool odd = (b & 1u) != 0u;
     float acc0[GU_R], acc1[GU_R];
-#pragma unroll
-    for (int i = 0; i < GU_R; ++i) acc0[i] = acc1[i] = 0.f;
-    // Steps of one stream word each, in the order (half, block, word): the codebook reads of step s + 1
-    // are issued between the products of step s, state by state, with fences that hold the order.
-    uint32_t raw[2][4][2], pr[2];
-    tq2_word_states(d[0], odd, 0, pr);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) tq2_state_gather(pr, j, book, raw[0][j]);
-    float x[64];
-#pragma unroll
-    for (int s = 0; s < 8 * GU_R; ++s) {
-        const int h = s / (4 * GU_R), i = (s / 4) % GU_R, ii = s % 4, n = s + 1;
-        if (s % (4 * GU_R) == 0) {
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const uint4 v = xb[16 * h + j];
-                x[4 * j] = gd_bits_f32(v.x);
-                x[4 * j + 1] = gd_bits_f32(v.y);
-                x[4 * j + 2] = gd_bits_f32(v.z);
-                x[4 * j + 3] = gd_bits_f32(v.w);
-            }
-        }
-        if (n < 8 * GU_R) tq2_word_states(d[(n / 4) % GU_R], odd, 4 * (n / (4 * GU_R)) + n % 4, pr);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (n < 8 * GU_R) tq2_state_gather(pr, j, book, raw[n & 1][j]);
-            __builtin_amdgcn_sched_barrier(0);
-            tq2_state_fma(raw[s & 1][j], x + 16 * ii + 4 * j, acc0[i], acc1[i]);
-            asm volatile("" : "+v"(acc0[i]), "+v"(acc1[i]));  // the products stay in their step
-        }
-    }
+    tq2_blocks_dot<GU_R>(d, odd, book, xb, acc0, acc1);
     float v[GU_R];
 #pragma unroll
     for (int i = 0; i < GU_R; ++i) {

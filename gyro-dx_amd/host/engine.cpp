@@ -1100,11 +1100,19 @@ class Engine {
             // (slot, block, half, row pair) items and 512 (row, slot) sums), about one group per
             // CU for a token. Layers of other types take the same kernels in their type-generic
             // form (_xg: rows through the expert table, each expert's types).
-            const uint32_t nb = E / 128, total = n * U * F, target = cus_or(256);
+            const uint32_t nb = E / 128, total = n * U * F;
+            // Two groups per CU (moe_decode_gu_gb / _xgb) once one would hold at least 7/8 of its 1024 items.
+            // Four layers replayed, us without and with: hidden 2560, F 640, top-10 2 tokens 151 -> 149 (GGUF 148
+            // 167 -> 160), 3 198 -> 166, 8 412 -> 357; 3072 / 768 / 16, 4 tokens 491 -> 418; below the line
+            // (1536 / 384 / 6, 2 and 6 tokens: 216 and 648 items) 85 -> 90 and 157 -> 159.
+            const bool batch = n > 1 && total * nb >= 896u * cus_or(256);
+            const uint32_t target = cus_or(256) * (batch ? 2u : 1u);
             const uint32_t rpg = std::max(1u, std::min({(total + target - 1) / target, F, 1024u / nb}));
             const uint32_t R = decode_down_rows();
             const uint32_t xt = generic ? L.xtab.srv : 0u;
-            dispatch_maybe_timed(bracket == 2, marks, generic ? "moe_decode_gu_xg" : "moe_decode_gu_g",
+            dispatch_maybe_timed(bracket == 2, marks,
+                                 generic ? (batch ? "moe_decode_gu_xgb" : "moe_decode_gu_xg")
+                                         : (batch ? "moe_decode_gu_gb" : "moe_decode_gu_g"),
                                  {B.logits, B.logits_off, NE, U, bits(L.scale), B.ids, B.ids_off, B.weights, B.weights_off, B.xh,
                                   B.xh_off, generic ? 0u : base_lo, generic ? 0u : base_hi, generic ? 0u : slot_stride,
                                   generic ? 0u : L.gate_bytes, codebook.srv, B.gu, B.gu_off, E, F, n, rpg, xt},
