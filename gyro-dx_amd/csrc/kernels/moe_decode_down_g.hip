@@ -3,7 +3,7 @@
 // dequant-GEMV of the down rows and the route-weighted combine (src/engine.zig:607-641).
 //
 // A group owns R consecutive output rows of one token for all U selected experts, so the
-// combine stays local and runs in slot order; the host picks R so that a token spans about one
+// combine stays local and runs in slot order; the host picks R so that a call spans few rounds of one
 // group per CU.
 //  - Item (slot k, block bb, half hf, row pair): each thread loads the expert id of its item,
 //    its inputs' values (below), then block bb of both rows straight from HBM (9 words each),
@@ -22,10 +22,10 @@
 // 4 weights_uav 5 weights_off 6 base_lo 7 base_hi 8 slot_stride 9 down_off 10 codebook_srv
 // 11 signs_srv (0xffffffff: none) 12 signs_off 13 out_uav (or its address in 58, 59) 14 out_off 15 E 16 F 17 n_used
 // 18 n_tok 19 R 20 n_expert 21 residual 22 res_uav 23 res_off (24 xtab_srv: the generic form).
-// Builds with DG_SHARED (moe_decode_down_gs, _xgs) add the shared expert's gated down rows,
+// Builds with DG_SHARED (moe_decode_down_gs, _xgs; _gs3, _xgs3 for R past 16) add the shared expert's gated down rows,
 // sigmoid(g[t]) * (W_sd[r] . a[t]) with a and g from moe_router_s: 25 row format (0 bf16, 1 Q8_0) 26 a_uav
 // 27 a_off (fp32 [n][SF]) 28 g_uav 29 g_off 30 w_srv 31 row bytes 32 SF (a multiple of 64 up to 1024);
-// R <= 16. A wave takes rows w and w + 8 of the group: their loads (at most 16 bytes x 2 a lane and row) go
+// R <= 8 DG_SH_ROWS. A wave takes rows w, w + 8 (and w + 16) of the group: their loads (16 bytes x 2 a lane and row) go
 // out before the routed blocks', and the products run while those are in flight, so the launch of
 // moe_decode_shared_down and its gap go. Measured, four
 // layers replayed at hidden 2560, F 640, top-10, Q8_0 of width 640: 1 token 116 -> 102 us, 2 tokens
@@ -47,6 +47,9 @@
 #ifndef DG_SHARED
 #define DG_SHARED 0  // 1: the shared expert's down rows too
 #endif
+#ifndef DG_SH_ROWS
+#define DG_SH_ROWS 2  // shared rows per wave
+#endif
 // Words loaded per block: TQ2_T's 34 bytes, or the widest type's 58 (whole words from the
 // block's first byte rounded down to a word; the arena's slack covers reads past the last row).
 #define DG_WORDS (DG_GENERIC ? 15 : 9)
@@ -66,7 +69,7 @@ DG_DEFINE(DG_PIPELINE, 512) {
     __shared__ float dred[2 * DG_ITEMS * 512];  // half dots by (slot, row, block, half)
     __shared__ float sw[DG_MAX_U];
 #if DG_SHARED
-    __shared__ float shs[16];  // W_sd[r0 + i] . a[t]
+    __shared__ float shs[8 * DG_SH_ROWS];  // W_sd[r0 + i] . a[t]
 #endif
 #if DG_GENERIC
     __shared__ gd_u32x4 xdesc[DG_MAX_EXPERTS];  // per expert {down lo, down hi, types, pad}
@@ -132,26 +135,26 @@ DG_DEFINE(DG_PIPELINE, 512) {
         svv[ps][1] = S[1];
     }
 #if DG_SHARED
-    // Rows `wave` and `wave` + 8 of the group (a wave past the last repeats it), columns 16 lane (Q8_0) or
+    // Rows `wave` + 8 i of the group (past the last one, that again), columns 16 lane (Q8_0) or
     // 8 lane and 512 + 8 lane (bf16); lanes past the last column read it again and multiply zeros.
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), SF = a.c[32];
     const bool q8 = a.c[25] != 0u;  // uniform
     const float sg_dot = gd_bits_f32(gd_global(gd_buf<const uint32_t>(a, a.c[28]) + a.c[29])[t]);
-    gd_u32x4 shw[2][2], shx[4];
-    uint32_t shd[2] = {0u, 0u};
+    gd_u32x4 shw[DG_SH_ROWS][2], shx[4];
+    uint32_t shd[DG_SH_ROWS] = {};
     bool shin[2];
     {
         const uint32_t *A = gd_buf<const uint32_t>(a, a.c[26]) + a.c[27] + (size_t)t * SF;
         const uint8_t *W = gd_buf<const uint8_t>(a, a.c[30]);
-        const uint8_t *row[2];
+        const uint8_t *row[DG_SH_ROWS];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) row[i] = W + (size_t)(r0 + min(wave + 8u * i, R - 1u)) * a.c[31];
+        for (int i = 0; i < DG_SH_ROWS; ++i) row[i] = W + (size_t)(r0 + min(wave + 8u * i, R - 1u)) * a.c[31];
         if (q8) {
             const uint32_t c = 16u * lane, col = c < SF ? c : SF - 16u;
             shin[0] = c < SF;
             shin[1] = false;
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < DG_SH_ROWS; ++i) {
                 shw[i][0] = *gd_global4(reinterpret_cast<const uint32_t *>(row[i] + col));
                 shw[i][1] = shw[i][0];
                 shd[i] = *(const __attribute__((address_space(1))) uint16_t *)(uintptr_t)(row[i] + SF + (col / 32u) * 2u);
@@ -164,7 +167,7 @@ DG_DEFINE(DG_PIPELINE, 512) {
                 const uint32_t c = 8u * (64u * m + lane), col = c < SF ? c : SF - 8u;
                 shin[m] = c < SF;
 #pragma unroll
-                for (int i = 0; i < 2; ++i) shw[i][m] = *gd_global4(reinterpret_cast<const uint32_t *>(row[i] + 2u * col));
+                for (int i = 0; i < DG_SH_ROWS; ++i)  shw[i][m] = *gd_global4(reinterpret_cast<const uint32_t *>(row[i] + 2u * col));
 #pragma unroll
                 for (int j = 0; j < 2; ++j) shx[2 * m + j] = *gd_global4(A + col + 4u * j);
             }
@@ -263,7 +266,7 @@ DG_DEFINE(DG_PIPELINE, 512) {
 #if DG_SHARED
     // The sums in shr_dots' order: a lane's columns, then the wave.
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < DG_SH_ROWS; ++i) {
         float p = 0.f;
         if (q8) {
             float v[16], d = 0.f;

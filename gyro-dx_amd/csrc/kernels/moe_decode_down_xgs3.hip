@@ -1,0 +1,7 @@
+// moe_decode_down_xgs with three shared rows per wave, for groups of 17 to 24 output rows.
+#define DG_MAX_ABLK 128
+#define DG_GENERIC 1
+#define DG_SHARED 1
+#define DG_SH_ROWS 3
+#define DG_PIPELINE moe_decode_down_xgs3
+#include "moe_decode_down_g.hip"

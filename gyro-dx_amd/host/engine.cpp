@@ -984,17 +984,28 @@ class Engine {
         }
         return 0;
     }
-    // Output rows of a moe_decode_down_g group: about one group per CU for a token, within its item and sum limits.
-    uint32_t decode_down_rows() const {
-        uint32_t R = std::max(1u, E / cus_or(256));
-        while (R > 1 && (E % R || U * (F / 128) * 2 * ((R + 1) / 2) > 1024 || R * U > 512)) --R;
-        return R;
+    // Output rows R of a moe_decode_down_g group, within its item and sum limits: the fewest rounds of one group
+    // per CU, a round costing a fixed part (ids, inputs and their rotation) and twice that per item of a thread. A
+    // token's R is E / 256, and a batch's the larger ones that save rounds: two tokens at hidden 2560, F 640,
+    // top-10 were two rounds of R 10 and are one of R 20 (two items). Four layers replayed, us (E / 256 -> this):
+    // that shape 2 tokens 128 -> 121, 4 205 -> 193, 8 363 -> 342; GGUF 148 4 tokens 277 -> 257; 1536 / 384 / 6
+    // 3 tokens 107 -> 86; 1024 / 256 / 2 8 tokens 149 -> 76. 3 tokens at R 16 or 20 (two rounds, two items)
+    // took 170 and 172 against 166 at R 10 (three rounds, one item).
+    uint32_t decode_down_rows(const Layer &L, uint32_t n) const {
+        uint32_t best = 1, best_cost = ~0u;
+        for (uint32_t R = 1; R <= (L.SF ? 24u : 32u); ++R) {
+            const uint32_t items = U * (F / 128) * 2 * ((R + 1) / 2);
+            if (E % R || items > 1024 || R * U > 512) continue;
+            const uint32_t cost = (E / R * n + cus_or(256) - 1) / cus_or(256) * (1 + 2 * ((items + 511) / 512));
+            if (cost < best_cost) best = R, best_cost = cost;
+        }
+        return best;
     }
     // Whether moe_decode_down_gs / _xgs takes the layer's shared down rows along (no moe_decode_shared_down):
-    // the shapes of the _g kernels whose groups keep one per CU (not _gl), at most two rows a wave, and rows
+    // the shapes of the _g kernels whose groups keep one per CU (not _gl), at most three rows a wave, and rows
     // of one 16-byte load (Q8_0) or two (bf16) a lane, held in registers beside the routed blocks.
     bool decode_folds_shared_down(const Layer &L) const {
-        if (!L.SF || decode_fused_shared(L) || L.SF > 1024 || L.sh_kind == GM_SHARED_F32 || decode_down_rows() > 16) return false;
+        if (!L.SF || decode_fused_shared(L) || L.SF > 1024 || L.sh_kind == GM_SHARED_F32) return false;
         return decode_generic_types(L) ? !decode_generic_tuned() : !decode_tuned_tq2() && U * (F / 128) <= 64;
     }
     uint32_t cus_or(uint32_t fallback) const { return cus ? cus : fallback; }
@@ -1108,7 +1119,7 @@ class Engine {
             const bool batch = n > 1 && total * nb >= 896u * cus_or(256);
             const uint32_t target = cus_or(256) * (batch ? 2u : 1u);
             const uint32_t rpg = std::max(1u, std::min({(total + target - 1) / target, F, 1024u / nb}));
-            const uint32_t R = decode_down_rows();
+            const uint32_t R = decode_down_rows(L, n);
             const uint32_t xt = generic ? L.xtab.srv : 0u;
             dispatch_maybe_timed(bracket == 2, marks,
                                  generic ? (batch ? "moe_decode_gu_xgb" : "moe_decode_gu_xg")
@@ -1117,8 +1128,8 @@ class Engine {
                                   B.xh_off, generic ? 0u : base_lo, generic ? 0u : base_hi, generic ? 0u : slot_stride,
                                   generic ? 0u : L.gate_bytes, codebook.srv, B.gu, B.gu_off, E, F, n, rpg, xt},
                                  (total + rpg - 1) / rpg);
-            const char *down = generic ? (folded ? "moe_decode_down_xgs" : "moe_decode_down_xg")
-                               : folded ? "moe_decode_down_gs"
+            const char *down = generic ? (!folded ? "moe_decode_down_xg" : R <= 16 ? "moe_decode_down_xgs" : "moe_decode_down_xgs3")
+                               : folded ? (R <= 16 ? "moe_decode_down_gs" : "moe_decode_down_gs3")
                                         : (U * (F / 128) <= 64 ? "moe_decode_down_g" : "moe_decode_down_gl");
             const SharedBufs &S = B.shared;
             dispatch_maybe_timed(bracket == 3, marks, down,
