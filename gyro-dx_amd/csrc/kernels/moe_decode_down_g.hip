@@ -167,7 +167,7 @@ DG_DEFINE(DG_PIPELINE, 512) {
                 const uint32_t c = 8u * (64u * m + lane), col = c < SF ? c : SF - 8u;
                 shin[m] = c < SF;
 #pragma unroll
-                for (int i = 0; i < DG_SH_ROWS; ++i)  shw[i][m] = *gd_global4(reinterpret_cast<const uint32_t *>(row[i] + 2u * col));
+                for (int i = 0; i < DG_SH_ROWS; ++i) shw[i][m] = *gd_global4(reinterpret_cast<const uint32_t *>(row[i] + 2u * col));
 #pragma unroll
                 for (int j = 0; j < 2; ++j) shx[2 * m + j] = *gd_global4(A + col + 4u * j);
             }
