@@ -14,7 +14,7 @@
 // Two builds of this source: moe_decode_gu (batch 1) copies the block's 128 activations into
 // registers at once, right after the barrier, so no read of them waits inside the dot (156
 // VGPRs: one group per compute unit, which batch 1's 256 groups need anyway); moe_decode_gu_b
-// (batches 2-8: 256 groups per token) reads them one half block at a time (64 VGPRs), so that
+// (batches: 256 groups per token) reads them one half block at a time (64 VGPRs), so that
 // up to four groups share a compute unit. Both compute the same products in the same order.
 // Expert e's rows are at base + e * slot_stride (+ proj_bytes for up): no table lookup.
 // Grid: x = F / 64, y = 2 * parts (projection-major), z = n_tok * 8; 512 threads.
