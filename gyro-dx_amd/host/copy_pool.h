@@ -28,7 +28,7 @@ class CopyPool {
     }
 
     // Hands a copy to the helpers in pieces of `piece` bytes (or makes it at once where there are none);
-    // both ranges stay untouched by the caller until finish().
+    // both ranges stay untouched by the caller until finish() or drop().
     void post(void *dst, const void *src, uint64_t bytes, uint64_t piece) {
         if (!start()) {
             std::memcpy(dst, src, bytes);
@@ -49,12 +49,31 @@ class CopyPool {
         run(lock);
         idle_.wait(lock, [this] { return running_ == 0; });
     }
+    // Drops what is still queued and returns once no helper copies: nothing posted is touched after it.
+    void drop() {
+        std::unique_lock<std::mutex> lock(mutex_);
+        queue_.clear();
+        idle_.wait(lock, [this] { return running_ == 0; });
+    }
+    // Around posts whose ranges the caller may free once it is told of an error: however the block is left,
+    // no copy is queued or running behind it.
+    class Scope {
+      public:
+        explicit Scope(CopyPool &pool) : pool_(pool) {}
+        ~Scope() { pool_.drop(); }
+        Scope(const Scope &) = delete;
+        Scope &operator=(const Scope &) = delete;
+
+      private:
+        CopyPool &pool_;
+    };
     // memcpy, from kParallelBytes on in pieces over all threads.
     void copy(void *dst, const void *src, uint64_t bytes) {
         if (bytes < kParallelBytes) {
             std::memcpy(dst, src, bytes);
             return;
         }
+        Scope scope(*this);
         post(dst, src, bytes, kPiece);
         finish();
     }

@@ -532,6 +532,7 @@ class Engine {
             part[i].ticket = submit();
         };
         Flags f;
+        CopyPool::Scope scope(copies);  // a wait or submission below may fail with copies into dst posted
         issue(0);
         for (uint32_t i = 0, issued = 1; i < parts; ++i) {
             for (; issued < parts && issued < i + kAhead; ++issued) issue(issued);
@@ -1497,6 +1498,7 @@ extern "C" int gm_create(const char *kernel_dir, uint32_t adapter, uint32_t max_
 
 extern "C" void gm_destroy(gm_engine *g) {
     if (!g) return;
+    g->e.copies.drop();  // before the staging slots go
     g->e.dev.deinit();
     delete g;
 }
