@@ -1025,18 +1025,17 @@ class Engine {
         explicit UnfusedPrefillScope(Engine *eng) : e(eng), was(eng->prefill_fused) { e->prefill_fused = false; }
         ~UnfusedPrefillScope() { e->prefill_fused = was; }
     };
-    // Clears the give-up word of the persistent GEMMs: set when a down unit stopped waiting for its
-    // tile's gate/up rows (the call's outputs are then invalid).
-    void clear_gemm_error() {
+    // Clears the words that f found set: the give-up word of the persistent GEMMs (a down unit stopped
+    // waiting for its tile's gate/up rows: the call's outputs are invalid) and the activation range flags (a
+    // fast-path kernel rounded an activation outside the binary16 range). Both stay set on the device
+    // until the host clears them, and a give-up leaves rows that a later kernel may find out of range.
+    void clear_flags(const Flags &f) {
         const uint32_t zero = 0;
-        upload(gemm_sched, 4, &zero, 4);
-    }
-    // Clears the activation range flags: set when a fast-path kernel rounded an activation outside the
-    // binary16 range.
-    void clear_range_flag() {
-        const uint32_t zero = 0;
-        upload(range_flag, 0, &zero, 4);
-        upload(meta, kMetaRangeFlag * 4, &zero, 4);
+        if (f.gemm_error) upload(gemm_sched, 4, &zero, 4);
+        if (f.range) {
+            upload(range_flag, 0, &zero, 4);
+            upload(meta, kMetaRangeFlag * 4, &zero, 4);
+        }
     }
 
     // MI355X decode path: router + rotation, routed gate/up, down + combine.
@@ -1382,19 +1381,18 @@ class Engine {
     }
 
     // One call through once(path), and again where its flags say that the outputs are not valid: after a
-    // give-up with two GEMM launches, after an activation outside the binary16 range on the generic path.
+    // give-up with two GEMM launches (whose own flags then decide), after an activation outside the
+    // binary16 range on the generic path.
     template <class Once>
     void run_checked(uint32_t path, Once &&once) {
         Flags f = once(path);
+        clear_flags(f);
         if (f.gemm_error) {
-            clear_gemm_error();
             UnfusedPrefillScope unfused{this};
             f = once(path);
+            clear_flags(f);
         }
-        if (f.range) {
-            clear_range_flag();
-            once(GM_PATH_GENERIC);
-        }
+        if (f.range) once(GM_PATH_GENERIC);
     }
 
     // The flag's table index for kernels of the fast paths (none on direct launches, whose
@@ -1629,8 +1627,7 @@ extern "C" int gm_run_bracketed(gm_engine *g, uint32_t path, uint32_t batch, uin
         *device_ms = dev;
         if (bracket_us) *bracket_us = br_n ? br / (double)br_n : 0.0;
         const Engine::Flags f = calls && Engine::fast_path(path) ? e.flags() : Engine::Flags{};
-        if (f.gemm_error) e.clear_gemm_error();
-        else if (f.range) e.clear_range_flag();
+        e.clear_flags(f);
         if (f.gemm_error)
             throw gyro::NativeError(-1, "a prefill GEMM unit gave up waiting for its tile's gate/up rows: the outputs of "
                                         "this run are invalid (gm_forward recomputes such calls with two GEMM launches)");
@@ -1675,8 +1672,7 @@ extern "C" int gm_run_stack(gm_engine *g, uint32_t path, uint32_t batch, uint32_
         *wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         *device_ms = dev;
         const Engine::Flags f = calls && Engine::fast_path(path) ? e.flags() : Engine::Flags{};
-        if (f.gemm_error) e.clear_gemm_error();
-        else if (f.range) e.clear_range_flag();
+        e.clear_flags(f);
         if (f.gemm_error)
             throw gyro::NativeError(-1, "a prefill GEMM unit gave up waiting for its tile's gate/up rows: the outputs of "
                                         "this run are invalid (gm_forward_stack recomputes such calls with two GEMM launches)");

@@ -135,6 +135,37 @@ def test_persistent_gemm_give_up_recomputes():
         eng.close()
 
 
+def test_give_up_with_an_activation_out_of_range():
+    """Both flag words set by one call (a spin limit of zero polls, a token whose rotated input exceeds binary16):
+    gm_forward returns the generic path's outputs, gm_run reports an error, and neither leaves a word
+    set: the call after it is the two-launch path's, bit for bit, not recomputed on the generic path."""
+    n = 16  # so few tiles that every unit starts at once, the down units ahead of their rows
+    L = synth.make_layer(1570, n_expert=8, n_used=2)
+    x = synth.make_tokens(1571, n, bf16=True)
+    far = x.copy()
+    far[n // 2, 0] = 2.0e6
+    ref_eng = make_engine(n, False)
+    try:
+        ref_eng.add_layer(L)
+        ref, ref_far = ref_eng.forward(0, x, PATH_PREFILL), ref_eng.forward(0, far, PATH_PREFILL)
+    finally:
+        ref_eng.close()
+    eng = make_engine(n, True, spin_limit=0)
+    try:
+        eng.add_layer(L)
+        print("persistent prefill GEMM, spin limit 0, one token out of range: gm_forward", flush=True)
+        np.testing.assert_array_equal(eng.forward(0, far, PATH_PREFILL).view(np.uint32), ref_far.view(np.uint32))
+        np.testing.assert_array_equal(eng.forward(0, x, PATH_PREFILL).view(np.uint32), ref.view(np.uint32))
+        print("  gm_run", flush=True)
+        eng.set_tokens(far)
+        with pytest.raises(RuntimeError, match="gave up waiting|binary16 range") as err:
+            eng.run(PATH_PREFILL, n, 1, [0])
+        print(f"  {err.value}", flush=True)
+        np.testing.assert_array_equal(eng.forward(0, x, PATH_PREFILL).view(np.uint32), ref.view(np.uint32))
+    finally:
+        eng.close()
+
+
 SMALL_SHAPES = [
     # E, F, experts, top-k, tokens, extra make_layer arguments
     (2048, 512, 256, 8, 128, {}),
