@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "copy_pool.h"
+#include "decode_split.h"
 #include "device.h"
 #include "gyro_moe.h"
 
@@ -985,22 +986,9 @@ class Engine {
         }
         return 0;
     }
-    // Output rows R of a moe_decode_down_g group, within its item and sum limits: the fewest rounds of one group
-    // per CU, a round costing a fixed part (ids, inputs and their rotation) and twice that per item of a thread. A
-    // token's R is E / 256, and a batch's the larger ones that save rounds: two tokens at hidden 2560, F 640,
-    // top-10 were two rounds of R 10 and are one of R 20 (two items). Four layers replayed, us (E / 256 -> this):
-    // that shape 2 tokens 128 -> 121, 4 205 -> 193, 8 363 -> 342; GGUF 148 4 tokens 277 -> 257; 1536 / 384 / 6
-    // 3 tokens 107 -> 86; 1024 / 256 / 2 8 tokens 149 -> 76. 3 tokens at R 16 or 20 (two rounds, two items)
-    // took 170 and 172 against 166 at R 10 (three rounds, one item).
+    // Output rows of a moe_decode_down_g group: the builds with the shared expert's rows take up to 24.
     uint32_t decode_down_rows(const Layer &L, uint32_t n) const {
-        uint32_t best = 1, best_cost = ~0u;
-        for (uint32_t R = 1; R <= (L.SF ? 24u : 32u); ++R) {
-            const uint32_t items = U * (F / 128) * 2 * ((R + 1) / 2);
-            if (E % R || items > 1024 || R * U > 512) continue;
-            const uint32_t cost = (E / R * n + cus_or(256) - 1) / cus_or(256) * (1 + 2 * ((items + 511) / 512));
-            if (cost < best_cost) best = R, best_cost = cost;
-        }
-        return best;
+        return gyro::decode_down_rows(E, F, U, n, cus_or(256), L.SF ? 24u : 32u);
     }
     // Whether moe_decode_down_gs / _xgs takes the layer's shared down rows along (no moe_decode_shared_down):
     // the shapes of the _g kernels whose groups keep one per CU (not _gl), at most three rows a wave, and rows
