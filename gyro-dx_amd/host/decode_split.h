@@ -5,6 +5,19 @@
 
 namespace gyro {
 
+// Blocks a lane of the batch kernels decodes at the tuned shape (n 2 to 8): 4 or 2, where the groups (E n / 32 and
+// E n / 16) fill at least 7/8 of whole rounds of one group per CU (at 256 CUs 2, 4 and 6 to 8 tokens at hidden
+// 2048, 4, 7 and 8 at 1024), else 0: moe_decode_gu_b and moe_decode_down, whose smaller groups balance better.
+// Four layers replayed, us without and with: hidden 2048, 2 tokens 81 -> 76, 4 112 -> 105, 6 145 -> 133,
+// 8 176 -> 154; forced at 3 tokens 96 -> 100, at 5 126 -> 147; hidden 1024, 4 tokens 82 -> 77, 8 114 -> 107.
+inline uint32_t decode_blocks_per_lane(uint32_t E, uint32_t n, uint32_t cus) {
+    for (uint32_t r : {4u, 2u}) {
+        const uint32_t groups = E * n / (8 * r), rounds = (groups + cus - 1) / cus;
+        if (8 * groups >= 7 * cus * rounds) return r;
+    }
+    return 0;
+}
+
 // Output rows R of a moe_decode_down_g group (E a multiple of R, at most max_rows and the kernel's limits of items
 // and sums): the fewest rounds of one group per CU, a round costing a fixed part (ids, inputs and their
 // rotation) and twice that per item of a thread. The larger R that save rounds are a batch's: two tokens at

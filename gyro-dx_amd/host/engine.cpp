@@ -974,18 +974,6 @@ class Engine {
     // Uniform TQ2_T layers take moe_decode_gu / moe_decode_down at their compile-time shape
     // (hidden 1024 or 2048, F 512, top-8), moe_decode_gu_g / moe_decode_down_g(l) otherwise.
     bool decode_tuned_tq2() const { return E % 1024 == 0 && F == 512 && U == 8 && parts <= 2; }
-    // Blocks a lane of the batch kernels decodes at the tuned shape: 4 or 2, where the groups (E n / 32 and
-    // E n / 16) fill at least 7/8 of whole rounds of 256 (2, 4 and 6 to 8 tokens at hidden 2048), else 0:
-    // moe_decode_gu_b and moe_decode_down, whose 2,048 smaller groups balance better.
-    // Four layers replayed, us without and with: hidden 2048, 2 tokens 81 -> 76, 4 112 -> 105, 6 145 -> 133,
-    // 8 176 -> 154; forced at 3 tokens 96 -> 100, at 5 126 -> 147; hidden 1024, 4 tokens 82 -> 77, 8 114 -> 107.
-    uint32_t decode_blocks_per_lane(uint32_t n) const {
-        for (uint32_t r : {4u, 2u}) {
-            const uint32_t groups = E * n / (8 * r), rounds = (groups + 255) / 256;
-            if (8 * groups >= 7 * 256 * rounds) return r;
-        }
-        return 0;
-    }
     // Output rows of a moe_decode_down_g group: the builds with the shared expert's rows take up to 24.
     uint32_t decode_down_rows(const Layer &L, uint32_t n) const {
         return gyro::decode_down_rows(E, F, U, n, cus_or(256), L.SF ? 24u : 32u);
@@ -1080,7 +1068,7 @@ class Engine {
                                                   slot_stride, 2 * L.gate_bytes, codebook.srv,
                                                   L.has_down_signs ? L.signs.srv : kNone, E, out_uav, out_off, E, F, U, n, parts,
                                                   NE, st.res_uav != kNone ? 1u : 0u, st.res_uav, st.res_off};
-                const uint32_t r = n == 1 ? 0u : decode_blocks_per_lane(n);
+                const uint32_t r = n == 1 ? 0u : gyro::decode_blocks_per_lane(E, n, cus_or(256));
                 if (r) {
                     const uint32_t rows = 8 * (64 / (E / 128)) * r / 2;  // gate/up rows of a group
                     dispatch_maybe_timed(bracket == 2, marks, r == 4 ? "moe_decode_gu_r4" : "moe_decode_gu_r2", gu,

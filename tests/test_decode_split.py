@@ -20,6 +20,17 @@ int main() {
 }
 """
 
+BLOCKS = r"""
+#include <cstdio>
+#include "decode_split.h"
+int main() {
+    for (unsigned cus : {256u, 304u, 64u, 32u})
+        for (unsigned E : {1024u, 2048u})
+            for (unsigned n = 2; n <= 8; ++n)
+                std::printf("%u %u %u %u\n", cus, E, n, gyro::decode_blocks_per_lane(E, n, cus));
+}
+"""
+
 
 def lines(tmp_path, program):
     src, exe = tmp_path / "split.cpp", tmp_path / "split"
@@ -50,3 +61,13 @@ def test_down_rows_examples(tmp_path):
     rows = {k[2:6]: k[6] for k in lines(tmp_path, DOWN) if k[0] == 256 and k[1] == 32}
     assert rows[2560, 640, 10, 1] == 10 and rows[2560, 640, 10, 2] == 20 and rows[2560, 640, 10, 3] == 10
     assert rows[1024, 256, 2, 8] == 32 and rows[3840, 768, 16, 1] == 8 and rows[256, 1024, 16, 1] == 1
+
+
+def test_blocks_per_lane(tmp_path):
+    """Four or two blocks where their groups fill 7/8 of whole rounds of the device's own units."""
+    got = {k[:3]: k[3] for k in lines(tmp_path, BLOCKS)}
+    for (cus, E, n), r in got.items():
+        fills = [b for b in (4, 2) if 8 * (E * n // (8 * b)) >= 7 * cus * -(-E * n // (8 * b) // cus)]
+        assert r == (fills[0] if fills else 0), (cus, E, n, r)
+    assert [got[256, 2048, n] for n in range(2, 9)] == [2, 0, 4, 0, 2, 4, 4]
+    assert [got[256, 1024, n] for n in range(2, 9)] == [0, 0, 2, 0, 0, 4, 4]
