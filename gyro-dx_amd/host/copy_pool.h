@@ -17,6 +17,7 @@ namespace gyro {
 class CopyPool {
   public:
     static constexpr uint64_t kPiece = 128u << 10;
+    static constexpr uint64_t kParallelBytes = 1u << 20;  // a copy from here on is worth waking the helpers
 
     ~CopyPool() {
         {
@@ -79,7 +80,6 @@ class CopyPool {
     }
 
   private:
-    static constexpr uint64_t kParallelBytes = 384u << 10;
     static constexpr unsigned kHelpers = 5;
 
     struct Piece {

@@ -455,32 +455,37 @@ class Engine {
     static uint32_t transfer_groups(uint32_t words) { return std::max(1u, (words + 4095) / 4096); }
 
     // Records the copy of at most kSlotBytes host bytes into a device buffer (a recording is open).
-    void record_upload(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes) {
+    void record_upload(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes, bool threads) {
         const uint32_t s = take_slot(), words = (uint32_t)(bytes / 4), at = (uint32_t)(s * (kSlotBytes / 4));
-        copies.copy(staging.mapped + s * kSlotBytes, src, bytes);
+        if (threads)
+            copies.copy(staging.mapped + s * kSlotBytes, src, bytes);
+        else
+            std::memcpy(staging.mapped + s * kSlotBytes, src, bytes);
         dispatch("transfer", {staging.uav, at, dst.uav, (uint32_t)(dst_off / 4), words}, transfer_groups(words));
-    }
-    // Size of the parts a transfer of `bytes` goes in: the host's copies and the link's overlap from part
-    // to part, but a part's submission costs the host about 8 us.
-    static uint64_t part_bytes(uint64_t bytes) {
-        const uint64_t p = (bytes / 6 + 4095) & ~uint64_t(4095);
-        return std::min(kSlotBytes, std::max<uint64_t>(p, 512u << 10));
     }
     // Copies host bytes into a device buffer. All but the last part go out in submissions of their own, so
     // that the host fills the next slot while the link moves this one; the last is left in an open
     // recording (begin_upload), submitted (upload_later: for data that only this stream reads before
     // the next wait) or submitted and waited for (upload). The source is read before any returns.
+    // Up to kThreadedUpload one thread copies, in parts of 1 to 2 MB, three where that holds them: waking the
+    // helpers for each part costs more than they take over, a submission costs the host 8 us, and the
+    // fourth one waits for the first (the context keeps three in flight). gm_set_tokens, us (one blocking transfer /
+    // parts of a sixth with helpers / this): 1.6 MB 195 / 222 / 193, 3.2 MB 318 / 348 / 300, 5 MB 380 / 402 / 350, 8 MB
+    // 479 / 489 / 456. Past it helpers and whole slots: 32 MB 993, one thread 1394.
+    static constexpr uint64_t kThreadedUpload = 8u << 20;
     void begin_upload(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes) {
         if (bytes % 4 || dst_off % 4) throw NativeError(-1, "upload must be word aligned");
         const uint8_t *s = static_cast<const uint8_t *>(src);
-        const uint64_t part = part_bytes(bytes);
+        const bool threads = bytes > kThreadedUpload;
+        const uint64_t third = (bytes / 3 + 4096) & ~uint64_t(4095);
+        const uint64_t part = threads ? kSlotBytes : std::min(kSlotBytes, std::max<uint64_t>(third, 1u << 20));
         for (; bytes > part; bytes -= part, s += part, dst_off += part) {
             dev.begin();
-            record_upload(dst, dst_off, s, part);
+            record_upload(dst, dst_off, s, part, threads);
             submit();
         }
         dev.begin();
-        if (bytes) record_upload(dst, dst_off, s, bytes);
+        if (bytes) record_upload(dst, dst_off, s, bytes, threads);
     }
     uint64_t upload_later(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes) {
         begin_upload(dst, dst_off, src, bytes);
@@ -499,6 +504,15 @@ class Engine {
     }
     Flags flags() const { return {status.words()[0], status.words()[1] | status.words()[2]}; }  // after the wait
 
+    // Size of the parts a download of `bytes` goes in: the host's copies and the link's overlap from part
+    // to part, but a part's submission costs the host about 8 us, and waking the helpers more than they take over
+    // of a few hundred KB: less than 1 MB is one part, copied by the caller (gm_read_outputs, us, blocking / parts of
+    // 512 KB with helpers / this: 384 KB 36 / 46 / 32, 520 KB 42 / 56 / 38, 768 KB 53 / 59 / 50; 1 MB 76 / 64 / 69).
+    static uint64_t part_bytes(uint64_t bytes) {
+        if (bytes < CopyPool::kParallelBytes) return kSlotBytes;
+        const uint64_t p = (bytes / 6 + 4095) & ~uint64_t(4095);
+        return std::min(kSlotBytes, std::max<uint64_t>(p, 512u << 10));
+    }
     // Ends the open recording with the copy of `bytes` of a device buffer to host memory (and, with
     // want_flags, of the flag words): the first part in this submission, later ones in their own,
     // kAhead ahead of the part whose copy out of its staging slot is handed on next. Returns the flags;

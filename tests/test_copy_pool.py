@@ -17,7 +17,7 @@ static int fail(const char *what, long a) { return std::printf("%s %ld\n", what,
 
 int main() {
     CopyPool pool;
-    for (long n : {0L, 1L, 131071L, 131072L, 393215L, 393216L, 393217L, 2097152L, 5000001L}) {
+    for (long n : {0L, 1L, 131071L, 131072L, 1048575L, 1048576L, 1048577L, 2097152L, 5000001L}) {
         std::vector<unsigned char> a(n), b(n);
         for (long i = 0; i < n; ++i) a[i] = (unsigned char)(i * 7 + n);
         pool.copy(b.data(), a.data(), n);

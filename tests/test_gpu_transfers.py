@@ -1,6 +1,6 @@
 """Host transfers in parts (set_tokens, read_outputs, gm_forward) at the sizes where their plan changes:
-one part below and at the threaded copy's threshold, two parts, a part of one slot, several slots, and
-a dozen parts and more, whose staging slots come round while copies are still queued. Rows that
+one part below the threaded copy's threshold and the parts at it, a part of one slot, several slots, one thread's
+and the helpers' uploads, and a dozen parts and more, whose staging slots come round while copies are still queued. Rows that
 went through the engine in one transfer each way must equal, bit for bit, the same rows sent eight at a
 time (32 KB, a single part)."""
 import numpy as np
@@ -20,8 +20,10 @@ def engine():
     eng.close()
 
 
-# 4 KB a token: 384 KB, one part of 512 KB, two parts, 4 MB, 12 MB in 2 MB slots, 24 MB in 13 parts.
-@pytest.mark.parametrize("n", [88, 96, 128, 136, 1032, 3080, 6200])
+# 4 KB a token. Downloads: one part copied by the caller up to 992 KB, two parts of 512 KB with the helpers at 1 MB, three,
+# 4 MB, 12 MB in 2 MB slots, 24 MB in 13 parts. Uploads: one part up to 1 MB, two, three of a third, 8 MB (one
+# thread's last) and 8 MB + 32 KB (helpers).
+@pytest.mark.parametrize("n", [88, 96, 128, 136, 248, 256, 264, 1032, 2048, 2056, 3080, 6200])
 def test_tokens_and_outputs_in_parts(engine, n):
     print(f"transfers: {n} tokens", flush=True)
     x = synth.make_tokens(5301 + n, n, 1024)
