@@ -381,9 +381,28 @@ class Engine {
         if (it == pipes.end()) throw NativeError(-1, std::string("pipeline missing: ") + name);
         return it->second;
     }
+    // The routed decode kernels' files: each layer shape takes a few of the two dozen builds, and loading one takes
+    // 0.4 ms (and unloading it as long), so gm_create leaves them to the first layer that dispatches them. No
+    // call loads one: it may be under capture.
+    std::map<std::string, std::string, std::less<>> decode_files;
+    bool loading = false;  // dispatches load their kernel and launch nothing
+    void load_decode_kernels(uint32_t il) {
+        struct Loading {
+            Engine *e;
+            explicit Loading(Engine *eng) : e(eng) { e->loading = true; }
+            ~Loading() { e->loading = false; }
+        } scope{this};
+        for (uint32_t n = 1; n <= 8; ++n)
+            if (decode_supported(layers.at(il), n)) ffn_decode(il, n, 0, 0, 0, 0);
+    }
 
     void dispatch_words(const char *name, const uint32_t *c, uint32_t count, uint32_t x, uint32_t y, uint32_t z) {
-        if (direct) {
+        if (loading) {
+            auto it = decode_files.find(name);
+            if (it == decode_files.end()) return;
+            pipes[it->first] = dev.pipeline(read_file(it->second));
+            decode_files.erase(it);
+        } else if (direct) {
             // Constants 56 to 59: the addresses of the caller's input and output (gd_buf_at), read by
             // the router and down kernels in the place of a table entry.
             uint32_t words[60] = {};
@@ -420,8 +439,11 @@ class Engine {
         while (dirent *ent = readdir(d)) {
             std::string name = ent->d_name;
             if (name.size() > 3 && name.compare(name.size() - 3, 3, ".co") == 0) {
-                std::vector<uint8_t> code = read_file(dir + "/" + name);
-                pipes[name.substr(0, name.size() - 3)] = dev.pipeline(code);
+                const std::string kernel = name.substr(0, name.size() - 3), file = dir + "/" + name;
+                if (kernel.compare(0, 11, "moe_decode_") == 0)
+                    decode_files[kernel] = file;
+                else
+                    pipes[kernel] = dev.pipeline(read_file(file));
             }
         }
         closedir(d);
@@ -844,6 +866,12 @@ class Engine {
         dev.begin();
         dev.wait(submit());
         layers.push_back(L);
+        try {
+            load_decode_kernels(il);
+        } catch (...) {
+            layers.pop_back();
+            throw;
+        }
         return il;
     }
 
