@@ -440,7 +440,7 @@ class Engine {
             std::string name = ent->d_name;
             if (name.size() > 3 && name.compare(name.size() - 3, 3, ".co") == 0) {
                 const std::string kernel = name.substr(0, name.size() - 3), file = dir + "/" + name;
-                if (kernel.compare(0, 11, "moe_decode_") == 0)
+                if (kernel.rfind("moe_decode_gu", 0) == 0 || kernel.rfind("moe_decode_down", 0) == 0)
                     decode_files[kernel] = file;
                 else
                     pipes[kernel] = dev.pipeline(read_file(file));
