@@ -227,35 +227,7 @@ DG_DEFINE(DG_PIPELINE, 512) {
         if (has_signs) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) { v[j] *= gd_bits_f32(svv[ps][0][j]); v[4 + j] *= gd_bits_f32(svv[ps][1][j]); }
-#pragma unroll
-            for (int w = 1; w < 8; w <<= 1)
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (!(j & w)) {
-                        const float lo = v[j], hi = v[j + w];
-                        v[j] = lo + hi;
-                        v[j + w] = lo - hi;
-                    }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float p1 = gd_dpp_f<0xB1>(v[j]);  // quad_perm [1,0,3,2]
-                v[j] = (l16 & 1u) ? p1 - v[j] : v[j] + p1;
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float p2 = gd_dpp_f<0x4E>(v[j]);  // quad_perm [2,3,0,1]
-                v[j] = (l16 & 2u) ? p2 - v[j] : v[j] + p2;
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float up4 = gd_dpp_f<0x104>(v[j]), dn4 = gd_dpp_f<0x114>(v[j]);  // row_shl:4, row_shr:4
-                v[j] = (l16 & 4u) ? dn4 - v[j] : v[j] + up4;
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float up8 = gd_dpp_f<0x108>(v[j]), dn8 = gd_dpp_f<0x118>(v[j]);  // row_shl:8, row_shr:8
-                v[j] = (l16 & 8u) ? dn8 - v[j] : v[j] + up8;
-            }
+            gd_fwht128_x8(v, l16);
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] *= GD_INV_SQRT128;
         }
