@@ -219,7 +219,10 @@ __device__ __forceinline__ void tq2_blocks_dot(const uint32_t (&d)[R][9], bool o
 #pragma unroll
     for (int i = 0; i < R; ++i) acc0[i] = acc1[i] = 0.f;
     // Steps of one stream word each, in the order (half, block, word): the codebook reads of step s + 1
-    // are issued between the products of step s, state by state, with fences that hold the order.
+    // are issued between the products of step s, state by state, with fences that hold the order. They hold the
+    // registers too: left to the compiler's own order the same sums took all 128 VGPRs and spilled
+    // (moe_decode_gu_r4 121 VGPRs -> 128 and 1,052 B of scratch a lane, _r2 102 -> 128 and 356 B); where no
+    // register is short the two orders ran alike.
     uint32_t raw[2][4][2], pr[2];
     tq2_word_states(d[0], odd, 0, pr);
 #pragma unroll
