@@ -59,4 +59,7 @@ def test_kernels_built():
     fast = {"moe_router", "moe_decode_gu", "moe_decode_gu_b", "moe_decode_down", "moe_dequant", "moe_prefill_router", "moe_prefill_router_w",
             "moe_prefill_topk", "moe_prefill_sort", "moe_prefill_gu", "moe_prefill_down", "moe_prefill_combine",
             "moe_stack_norm", "moe_decode_gu_x", "moe_decode_gu_xb", "moe_decode_down_x", "moe_decode_down_xb", "moe_decode_down_g", "moe_decode_gu_g", "moe_decode_gu_xg", "moe_decode_down_xg", "moe_prefill_gu_x", "moe_prefill_down_x", "gd_table_set"}
+    fast |= {"moe_decode_gu_r2", "moe_decode_gu_r4", "moe_decode_down_r2", "moe_decode_down_r4", "moe_decode_gu_gb",
+             "moe_decode_gu_xgb", "moe_decode_down_gl", "moe_decode_down_gs", "moe_decode_down_gs3", "moe_decode_down_xgs",
+             "moe_decode_down_xgs3", "moe_router_s", "moe_decode_shared_down", "transfer"}
     assert reference | fast <= kernels, (reference | fast) - kernels

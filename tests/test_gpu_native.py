@@ -170,6 +170,43 @@ def test_dispatch_contract(ctx):
     native.check(L.gd_release_pipeline(ctx, pipe, TIMEOUT))
 
 
+def test_table_entries_set_on_a_stream(ctx):
+    """gd_table_set points table entries at addresses known only when the work is queued (gd_dispatch_on): the next
+    dispatch copies between memory that no entry named before. An index past the table is skipped."""
+    L = native.lib()
+    pipes = {}
+    for name in ("gd_table_set", "transfer"):
+        pipes[name] = C.c_void_p()
+        native.check(L.gd_create_pipeline(ctx, code(name), len(code(name)), C.byref(pipes[name])))
+    entries = []
+    for _ in range(2):
+        h, info = C.c_void_p(), native.BufferInfo()
+        native.check(L.gd_wrap_memory(ctx, None, 0, C.byref(h), C.byref(info)), "gd_wrap_memory")
+        entries.append((h, info.uav_index))
+    host, hinfo = make_resource(ctx, 4096, 1)
+    dev, dinfo = make_resource(ctx, 4096, 0)
+    data = np.arange(1024, dtype=np.uint32) * 3 + 1
+    C.memmove(hinfo.mapped, data.ctypes.data, 4096)
+    words = [3]
+    for index, address in ((entries[0][1], hinfo.gpu_address or hinfo.mapped), (1 << 16, dinfo.gpu_address),
+                           (entries[1][1], dinfo.gpu_address)):
+        words += [index, address & 0xFFFFFFFF, address >> 32]
+    native.check(L.gd_dispatch_on(ctx, pipes["gd_table_set"], (C.c_uint32 * 10)(*words), 10, 1, 1, 1, None))
+    copy = (C.c_uint32 * 5)(entries[0][1], 0, entries[1][1], 0, 1024)
+    native.check(L.gd_dispatch_on(ctx, pipes["transfer"], copy, 5, 1, 1, 1, None))
+    native.check(L.gd_begin(ctx, TIMEOUT))  # a submission behind both, to wait for
+    ticket = C.c_uint64()
+    native.check(L.gd_submit(ctx, C.byref(ticket)))
+    native.check(L.gd_wait_compute(ctx, ticket, TIMEOUT))
+    back = np.zeros(1024, np.uint32)
+    native.check(L.gd_readback(ctx, dev, 0, 4096, back.ctypes.data, TIMEOUT))
+    np.testing.assert_array_equal(back, data)
+    for h in (dev, host, entries[0][0], entries[1][0]):
+        native.check(L.gd_release_buffer(ctx, h, TIMEOUT))
+    for p in pipes.values():
+        native.check(L.gd_release_pipeline(ctx, p, TIMEOUT))
+
+
 def test_stream_file_ranges(ctx):
     """src/native.zig:72-117: raw ranges of a file land in a buffer and read back equal."""
     L = native.lib()
