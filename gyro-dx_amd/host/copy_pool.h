@@ -1,7 +1,7 @@
 // Host copies between a caller's pageable memory and the engine's pinned staging slots, split over a few
 // threads: one thread moves 8-10 GB/s (page faults of a fresh output included), a sixth of the host
-// link. The helpers belong to one engine: they are started by its first large copy, sleep between
-// calls and are joined with it.
+// link. The helpers belong to one engine: they are started with its buffers where its calls can be
+// large, sleep between calls and are joined with it.
 #pragma once
 #include <condition_variable>
 #include <cstdint>
@@ -26,6 +26,20 @@ class CopyPool {
         }
         wake_.notify_all();
         for (std::thread &t : threads_) t.join();
+    }
+
+    // Starts the helpers, once (the first post does it at the latest); false where the system gives no thread.
+    bool start() {
+        if (!tried_) {
+            tried_ = true;
+            const unsigned cpus = std::thread::hardware_concurrency();
+            const unsigned n = cpus > kHelpers ? kHelpers : (cpus > 1 ? cpus - 1 : 0);
+            try {
+                for (unsigned i = 0; i < n; ++i) threads_.emplace_back([this] { helper(); });
+            } catch (const std::system_error &) {
+            }
+        }
+        return !threads_.empty();
     }
 
     // Hands a copy to the helpers in pieces of `piece` bytes (or makes it at once where there are none);
@@ -87,20 +101,6 @@ class CopyPool {
         const void *src;
         uint64_t bytes;
     };
-
-    // The helpers, at the first large copy; false where the system gives no thread.
-    bool start() {
-        if (!tried_) {
-            tried_ = true;
-            const unsigned cpus = std::thread::hardware_concurrency();
-            const unsigned n = cpus > kHelpers ? kHelpers : (cpus > 1 ? cpus - 1 : 0);
-            try {
-                for (unsigned i = 0; i < n; ++i) threads_.emplace_back([this] { helper(); });
-            } catch (const std::system_error &) {
-            }
-        }
-        return !threads_.empty();
-    }
 
     // Takes pieces until none is queued (the lock is held on entry and return, not while copying).
     void run(std::unique_lock<std::mutex> &lock) {

@@ -659,6 +659,8 @@ class Engine {
 
     void allocate_activations() {
         const uint64_t T = max_tok, f = 4;
+        // Five threads take 0.1 to 0.15 ms to start: not within the first call.
+        if (T * E * f >= CopyPool::kParallelBytes) copies.start();
         x_in = dev.buffer(T * E * f, Kind::device);
         router_out = dev.buffer(2 * T * NE * f, Kind::device);  // two logit planes of max_tok rows
         ids = dev.buffer(T * U * 4, Kind::device);
