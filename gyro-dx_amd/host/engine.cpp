@@ -489,18 +489,18 @@ class Engine {
     // that the host fills the next slot while the link moves this one; the last is left in an open
     // recording (begin_upload), submitted (upload_later: for data that only this stream reads before
     // the next wait) or submitted and waited for (upload). The source is read before any returns.
-    // Up to kThreadedUpload one thread copies, in parts of 1 to 2 MB, three where that holds them: waking the
-    // helpers for each part costs more than they take over, a submission costs the host 8 us, and the
-    // fourth one waits for the first (the context keeps three in flight). gm_set_tokens, us (one blocking transfer /
-    // parts of a sixth with helpers / this): 1.6 MB 195 / 222 / 193, 3.2 MB 318 / 348 / 300, 5 MB 380 / 402 / 350, 8 MB
-    // 479 / 489 / 456. Past it helpers and whole slots: 32 MB 993, one thread 1394.
-    static constexpr uint64_t kThreadedUpload = 8u << 20;
+    // What three slots hold the caller copies by itself: waking the helpers for each part costs more than they take
+    // over. It goes in one part up to 1 MB, two up to 2 and three past that: a submission costs the host 8 us, and
+    // a fourth one waits for the first (the context keeps three in flight). gm_set_tokens, us (one blocking
+    // transfer / parts of a sixth with helpers / this): 1.6 MB 193 / 222 / 181, 3.2 MB 318 / 348 / 298, 5 MB
+    // 380 / 402 / 353. Past it helpers and whole slots: 8 MB 478 / 489 / 447, 32 MB 1735 / 1029 / 993 (1394 alone).
+    static constexpr uint64_t kThreadedUpload = 3 * kSlotBytes;
     void begin_upload(const Buffer &dst, uint64_t dst_off, const void *src, uint64_t bytes) {
         if (bytes % 4 || dst_off % 4) throw NativeError(-1, "upload must be word aligned");
         const uint8_t *s = static_cast<const uint8_t *>(src);
         const bool threads = bytes > kThreadedUpload;
-        const uint64_t third = (bytes / 3 + 4096) & ~uint64_t(4095);
-        const uint64_t part = threads ? kSlotBytes : std::min(kSlotBytes, std::max<uint64_t>(third, 1u << 20));
+        const uint64_t parts = std::max<uint64_t>(1, std::min<uint64_t>(3, (bytes + (1u << 20) - 1) >> 20));
+        const uint64_t part = threads ? kSlotBytes : std::min(kSlotBytes, (bytes / parts + 4095) & ~uint64_t(4095));
         for (; bytes > part; bytes -= part, s += part, dst_off += part) {
             dev.begin();
             record_upload(dst, dst_off, s, part, threads);
@@ -550,10 +550,6 @@ class Engine {
         static_assert(kAhead + kBatch <= kSlots, "slots of a download");
         const uint64_t step = part_bytes(bytes);
         const uint32_t parts = (uint32_t)((bytes + step - 1) / step);
-        // All threads on one part until it is out; from a dozen parts on one thread on each, which a fresh
-        // output in 2 MB pages needs: a page is cleared by the first thread that touches it while
-        // the others wait (32 MB: 2.3 ms in small pieces, 0.75 ms in whole parts).
-        const uint64_t piece = parts >= 12 ? step : CopyPool::kPiece;
         std::vector<Part> part(parts);
         auto issue = [&](uint32_t i) {
             if (i) dev.begin();
@@ -586,7 +582,7 @@ class Engine {
             if (parts == 1) {
                 copies.copy(to, from, part[i].bytes);
             } else {
-                copies.post(to, from, part[i].bytes, piece);
+                copies.post(to, from, part[i].bytes);
                 if ((i + 1) % kBatch == 0 || i + 1 == parts) copies.finish();
             }
         }

@@ -32,7 +32,7 @@ int main() {
             CopyPool::Scope scope(pool);
             for (long i = 0; i < kParts; ++i) {
                 if (i == posted) throw std::runtime_error("wait");
-                pool.post(dst.get() + i * kPart, src.get() + i * kPart, kPart, round & 1 ? kPart : CopyPool::kPiece);
+                pool.post(dst.get() + i * kPart, src.get() + i * kPart, round & 1 ? kPart : CopyPool::kPiece);
             }
             pool.finish();
         } catch (const std::runtime_error &) {

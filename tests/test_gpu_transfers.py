@@ -21,9 +21,9 @@ def engine():
 
 
 # 4 KB a token. Downloads: one part copied by the caller up to 992 KB, two parts of 512 KB with the helpers at 1 MB, three,
-# 4 MB, 12 MB in 2 MB slots, 24 MB in 13 parts. Uploads: one part up to 1 MB, two, three of a third, 8 MB (one
-# thread's last) and 8 MB + 32 KB (helpers).
-@pytest.mark.parametrize("n", [88, 96, 128, 136, 248, 256, 264, 1032, 2048, 2056, 3080, 6200])
+# 4 MB, 12 MB in 2 MB slots, 24 MB in 13 parts. Uploads: one part up to 1 MB, two up to 2 MB, three up to 6 MB (the last
+# that the caller copies), whole slots with the helpers from there on.
+@pytest.mark.parametrize("n", [88, 96, 128, 136, 248, 256, 264, 512, 520, 1032, 1536, 1544, 3080, 6200])
 def test_tokens_and_outputs_in_parts(engine, n):
     print(f"transfers: {n} tokens", flush=True)
     x = synth.make_tokens(5301 + n, n, 1024)
